@@ -313,6 +313,31 @@ int ir_paged_attention_masked(const void* q, int64_t q_b_stride, int64_t q_s_str
                               ir_stream_t stream);
 
 /*
+ * ir_paged_attention_masked that may cut the keys of a call with too few
+ * workgroups for the device into parts, their fp32 partial rows in `workspace`
+ * (16-byte aligned scratch, nothing kept in it between calls; null: one part).
+ * It uses as many parts as pay and `workspace_bytes` holds;
+ * ir_paged_attention_masked_workspace_size gives the bytes for all of them (0:
+ * one part is best), at most 256 MiB.
+ */
+int64_t ir_paged_attention_masked_workspace_size(int batch, int seq_q, int seq_k,
+                                                 int num_q_heads, int num_kv_heads,
+                                                 int head_dim, int dtype, int mask_dtype,
+                                                 int64_t mask_t_stride);
+int ir_paged_attention_masked_ws(const void* q, int64_t q_b_stride, int64_t q_s_stride,
+                                 int64_t q_h_stride, const void* k_cache, const void* v_cache,
+                                 int64_t cache_slot_stride, int64_t cache_head_stride,
+                                 int64_t num_slots, const int64_t* gather_slots,
+                                 int64_t gs_b_stride, int64_t gs_t_stride, const void* mask,
+                                 int64_t mask_b_stride, int64_t mask_s_stride,
+                                 int64_t mask_t_stride, int mask_dtype, void* out,
+                                 int64_t out_b_stride, int64_t out_s_stride,
+                                 int64_t out_h_stride, int batch, int seq_q, int seq_k,
+                                 int num_q_heads, int num_kv_heads, int head_dim, float scale,
+                                 int dtype, int32_t* err_flags, const int32_t* run_if,
+                                 void* workspace, int64_t workspace_bytes, ir_stream_t stream);
+
+/*
  * Block tables from the reference engine's own decode metadata, so unchanged
  * callers of the seam reach the block-table decode kernels. The reference's
  * eager decode passes gather_slots[i, p] = bt_i[p / bs] * bs + p % bs (0 past

@@ -395,12 +395,20 @@ def paged_attention_masked(
         require_device(q, run_if)
         if run_if.dtype != torch.int32 or run_if.numel() < 1:
             raise RuntimeError("paged_attention_masked: run_if must be an int32 device tensor")
-    rc = lib().ir_paged_attention_masked(
+    ws = None
+    # (a call of up to 192 keys is never split; a gated one of few columns needs no workspace)
+    if t > 192 and (run_if is None or sq * (hq // h_kv) > 32):
+        need = lib().ir_paged_attention_masked_workspace_size(
+            b, sq, t, hq, h_kv, d, dtype_code(q.dtype), dtype_code(m.dtype), m.stride(3))
+        if need > 0:
+            ws = torch.empty(need, dtype=torch.uint8, device=dev)
+    rc = lib().ir_paged_attention_masked_ws(
         ptr(q), q.stride(0), q.stride(1), q.stride(2), ptr(k_cache), ptr(v_cache),
         k_cache.stride(0), k_cache.stride(1), k_cache.shape[0], ptr(gather_slots),
         gather_slots.stride(0), gather_slots.stride(1), ptr(m), m.stride(0), m.stride(2),
         m.stride(3), dtype_code(m.dtype), ptr(out), out.stride(0), out.stride(1), out.stride(2),
-        b, sq, t, hq, h_kv, d, float(scale), dtype_code(q.dtype), ptr(err_flags), ptr(run_if), stream_ptr(dev),
+        b, sq, t, hq, h_kv, d, float(scale), dtype_code(q.dtype), ptr(err_flags), ptr(run_if),
+        ptr(ws), 0 if ws is None else ws.numel(), stream_ptr(dev),
     )
     check(rc, "ir_paged_attention_masked")
     return out

@@ -454,6 +454,61 @@ def test_masked_fully_masked_row_is_uniform_and_bad_slot_flagged():
     assert err.item() == ERR_GATHER_RANGE
 
 
+@pytest.mark.parametrize("b,sq,t,h_kv,n_rep,d,dtype,mask_dtype", [
+    (1, 4, 1, 4, 7, 128, torch.bfloat16, torch.bfloat16),     # 28 columns: the narrow kernel, one key
+    (3, 1, 1003, 2, 7, 64, torch.float32, torch.float32),     # split, ragged last 16 keys
+    (2, 1, 2048, 4, 7, 128, torch.float16, torch.float32),    # split, whole tiles
+    (1, 5, 63, 4, 7, 128, torch.bfloat16, torch.bfloat16),    # 35 columns: the wide kernel, one ragged tile
+    (1, 19, 64, 4, 7, 128, torch.float16, torch.float16),     # 133 columns: a second workgroup of 5
+    (1, 40, 577, 2, 7, 64, torch.bfloat16, torch.bfloat16),   # split wide, ragged, head_dim 64
+    (2, 37, 700, 4, 7, 128, torch.bfloat16, torch.float32),   # fp32 mask read per lane
+    (1, 70, 321, 2, 4, 128, torch.bfloat16, torch.bfloat16),  # 4 heads a token: 16-bit mask read per lane
+    (1, 130, 200, 1, 1, 64, torch.float16, torch.float16),    # one head a token
+    (1, 27, 130, 1, 5, 128, torch.bfloat16, torch.bfloat16),  # 5 heads: 27 tokens in a workgroup
+    (1, 9, 4200, 1, 40, 64, torch.bfloat16, torch.bfloat16),  # 40 heads a token
+])
+@pytest.mark.parametrize("strided", [False, True])
+def test_masked_kernels_at_their_edges(b, sq, t, h_kv, n_rep, d, dtype, mask_dtype, strided):
+    """Random masks (zeros, finite biases, finfo.min, one row wholly masked) and a slot
+    outside the pool, over both kernels and their splits; ``strided``: key stride 2 in the
+    mask (the narrow kernel) and in the slots. The gated call gives the same bits."""
+    g = torch.Generator().manual_seed(sq * t)
+    slots_n = 1500
+    kc = torch.randn(slots_n, h_kv, d, generator=g).to(dtype)
+    vc = torch.randn(slots_n, h_kv, d, generator=g).to(dtype)
+    gs = torch.randint(0, slots_n, (b, t), generator=g)
+    low = max(torch.finfo(mask_dtype).min, torch.finfo(dtype).min)
+    mask = torch.randn(b, 1, sq, t, generator=g).to(mask_dtype)
+    mask[torch.rand(b, 1, sq, t, generator=g) < 0.6] = low
+    mask[0, 0, 0, :] = low
+    q = torch.randn(b, sq, h_kv * n_rep, d, generator=g).to(dtype)
+    # the oracle without the key whose slot is bad (t = 1 keeps its only key)
+    keep = torch.ones(t, dtype=torch.bool)
+    bad = t // 2 if t > 1 else None
+    if bad is not None:
+        keep[bad] = False
+    ref = O.paged_attention_naive(q.float(), kc.float(), vc.float(), gs[:, keep], mask[..., keep].float(), d**-0.5,
+                                  n_rep)
+    if bad is not None:
+        gs[:, bad] = slots_n + 3
+    gs, mask = gs.to(DEV), mask.to(DEV)
+    if strided:
+        gs = torch.stack([gs, gs], -1)[..., 0]
+        mask = torch.stack([mask, mask], -1)[..., 0]
+    args = (q.to(DEV), kc.to(DEV), vc.to(DEV), gs, mask, d**-0.5)
+    err = _err()
+    out = kernels.paged_attention_masked(*args, err_flags=err)
+    assert (out.float().cpu() - ref).abs().max().item() <= TOL[dtype]
+    assert err.item() == (ERR_GATHER_RANGE if bad is not None else 0)
+    gate = torch.ones(1, dtype=torch.int32, device=DEV)
+    gated = torch.full_like(out, 7.0)
+    assert torch.equal(kernels.paged_attention_masked(*args, out=gated, run_if=gate), out)
+    gate.zero_()
+    gated.fill_(7.0)
+    kernels.paged_attention_masked(*args, out=gated, run_if=gate)
+    assert bool((gated == 7.0).all())
+
+
 def test_config_table_is_consistent():
     for name, cfg in DECODE_CONFIGS.items():
         assert cfg.num_q_heads % cfg.num_kv_heads == 0, name
