@@ -338,6 +338,31 @@ int ir_paged_attention_masked_ws(const void* q, int64_t q_b_stride, int64_t q_s_
                                  void* workspace, int64_t workspace_bytes, ir_stream_t stream);
 
 /*
+ * A decode step's fixed-shape inputs from one staging buffer (device, 8-byte
+ * aligned): int64 [num_rows][2] (cached tokens, last token), then int32
+ * [num_rows][width] block tables; rows [num_rows, bucket) repeat row 0
+ * (build_decode_static_inputs, infrared/engine/cuda_graph.py:105-155). Writes
+ * ids, positions, write_slots [bucket] int64, gather_slots [bucket][t_max] int64
+ * (0 past the context), mask [bucket][t_max] of mask_dtype (0, finfo.min past the
+ * context), block_tables [bucket][width] and context_lens [bucket] int32. Every
+ * row's cached tokens must lie in [0, t_max), and width * block_size cover t_max.
+ */
+int ir_decode_inputs(const void* staging, int num_rows, int bucket, int width, int block_size,
+                     int t_max, int mask_dtype, int64_t* ids, int64_t* positions,
+                     int64_t* write_slots, int64_t* gather_slots, void* mask,
+                     int32_t* block_tables, int32_t* context_lens, ir_stream_t stream);
+
+/*
+ * Slots of a packed step's new tokens: token t of sequence b (cu_seqlens_q[b] <=
+ * t < cu_seqlens_q[b + 1]) at position p = num_cached[b] + t - cu_seqlens_q[b]
+ * gets block_tables[b][p / bs] * bs + p % bs (infrared/engine/paged_engine.py:
+ * 621-625); -1 past the table.
+ */
+int ir_packed_write_slots(const int32_t* block_tables, int64_t bt_stride, int width,
+                          const int32_t* num_cached, const int32_t* cu_seqlens_q, int num_seqs,
+                          int total, int block_size, int64_t* write_slots, ir_stream_t stream);
+
+/*
  * Block tables from the reference engine's own decode metadata, so unchanged
  * callers of the seam reach the block-table decode kernels. The reference's
  * eager decode passes gather_slots[i, p] = bt_i[p / bs] * bs + p % bs (0 past

@@ -5,7 +5,7 @@ Same API as the reference module:
 - ``default_buckets`` / ``pick_bucket`` (``infrared/engine/cuda_graph.py:58-81``);
 - ``build_decode_static_inputs`` (``:105-155``): fixed-shape inputs for a batch
   bucket, pad-by-repeating row 0, key axis padded to ``t_max``. Built
-  vectorised on the device instead of a Python loop over ``B * ctx`` tokens, and
+  by one kernel (``ir_decode_inputs``) instead of a Python loop over ``B * ctx`` tokens, and
   carrying the ``block_tables``/``context_lens`` the HIP decode kernel reads;
 - ``HipGraphDecoder`` (in place of ``CudaGraphDecoder``, ``:170-287``): one
   captured graph per bucket sharing one memory pool; ``decode()`` copies the
@@ -27,10 +27,12 @@ from __future__ import annotations
 from collections.abc import Callable, Sequence
 from dataclasses import dataclass
 
+import numpy as np
 import torch
 
 from infrared_amd import metadata
-from infrared_amd.paged_kv_cache import PagedContext, PagedKVPool
+from infrared_amd._lib import check, dtype_code, lib, ptr, stream_ptr
+from infrared_amd.paged_kv_cache import PagedContext, PagedKVPool, to_device
 
 
 def default_buckets(max_num_seqs: int) -> tuple[int, ...]:
@@ -88,19 +90,26 @@ def build_decode_static_inputs(
     Row ``i``'s new token is at position ``num_cached[i]`` (written to
     ``slot(bt_i, num_cached[i])``) and attends ``[0, num_cached[i]]``.
     """
-    b = len(last_tokens)
-    if not 0 < b <= bucket_b:
-        raise ValueError(f"need 0 < b ({b}) <= bucket_b ({bucket_b})")
+    device = torch.device(device)
+    b = _check_rows(num_cached, last_tokens, bucket_b, t_max)
     width = metadata.blocks_for(t_max, block_size)
+    if device.type == "cuda" and dtype in _MASK_DTYPES and bucket_b < 65536:
+        out = DecodeInputs(
+            ids=torch.empty(bucket_b, 1, dtype=torch.long, device=device),
+            positions=torch.empty(bucket_b, 1, dtype=torch.long, device=device),
+            write_slots=torch.empty(bucket_b, dtype=torch.long, device=device),
+            gather_slots=torch.empty(bucket_b, t_max, dtype=torch.long, device=device),
+            mask=torch.empty(bucket_b, 1, 1, t_max, dtype=dtype, device=device),
+            block_tables=torch.empty(bucket_b, width, dtype=torch.int32, device=device),
+            context_lens=torch.empty(bucket_b, dtype=torch.int32, device=device),
+        )
+        _fill_inputs(out, block_tables, num_cached, last_tokens, block_size)
+        return out
     rows = [i if i < b else 0 for i in range(bucket_b)]
-    ctx = [num_cached[j] + 1 for j in rows]
-    for c in ctx:
-        if c > t_max:
-            raise ValueError(f"context_len {c} exceeds t_max {t_max}")
     bt = metadata.block_tables_tensor(
         [list(block_tables[j])[:width] for j in rows], device, width
     )
-    cl = torch.tensor(ctx, dtype=torch.int32, device=device)
+    cl = torch.tensor([num_cached[j] + 1 for j in rows], dtype=torch.int32, device=device)
     nc = torch.tensor([num_cached[j] for j in rows], dtype=torch.long, device=device)
     ids = torch.tensor([[last_tokens[j]] for j in rows], dtype=torch.long, device=device)
     return DecodeInputs(
@@ -112,6 +121,41 @@ def build_decode_static_inputs(
         block_tables=bt,
         context_lens=cl,
     )
+
+
+_MASK_DTYPES = (torch.float32, torch.float16, torch.bfloat16)
+
+
+def _check_rows(num_cached: Sequence[int], last_tokens: Sequence[int], bucket_b: int, t_max: int) -> int:
+    """The rows of a step that fits ``(bucket_b, t_max)``; raises otherwise."""
+    b = len(last_tokens)
+    if not 0 < b <= bucket_b:
+        raise ValueError(f"need 0 < b ({b}) <= bucket_b ({bucket_b})")
+    for n in num_cached[:b]:
+        if n < 0:
+            raise ValueError(f"num_cached {n} is negative")
+        if n + 1 > t_max:
+            raise ValueError(f"context_len {n + 1} exceeds t_max {t_max}")
+    return b
+
+
+def _fill_inputs(out: DecodeInputs, block_tables: Sequence[Sequence[int]], num_cached: Sequence[int],
+                 last_tokens: Sequence[int], block_size: int) -> None:
+    """Writes a step's inputs into ``out`` (device tensors, contiguous): one
+    host array, one copy, one launch (``ir_decode_inputs``)."""
+    b, (bucket_b, width) = len(last_tokens), out.block_tables.shape
+    host = np.zeros(4 * b + b * width, dtype=np.int32)
+    rows = host[: 4 * b].view(np.int64).reshape(b, 2)
+    rows[:, 0] = num_cached[:b]
+    rows[:, 1] = last_tokens
+    metadata.fill_tables(host[4 * b :].reshape(b, width), [list(block_tables[j])[:width] for j in range(b)])
+    dev = out.mask.device
+    staging = to_device(host, dev)
+    check(lib().ir_decode_inputs(
+        ptr(staging), b, bucket_b, width, block_size, out.mask.shape[-1], dtype_code(out.mask.dtype), ptr(out.ids),
+        ptr(out.positions), ptr(out.write_slots), ptr(out.gather_slots), ptr(out.mask), ptr(out.block_tables),
+        ptr(out.context_lens), stream_ptr(dev),
+    ), "ir_decode_inputs")
 
 
 @dataclass(slots=True)
@@ -167,14 +211,18 @@ class HipGraphDecoder:
         """Advance the running set one token by graph replay; returns the first ``b`` rows."""
         b = len(last_tokens)
         bucket = pick_bucket(b, self.buckets)
-        inp = build_decode_static_inputs(
-            block_tables, num_cached, last_tokens, bucket, self.t_max, self.block_size,
-            self.device, self.dtype,
-        )
-        if bucket not in self._graphs:
-            self._capture(bucket, inp)
+        if bucket in self._graphs and self.dtype in _MASK_DTYPES and bucket < 65536:
+            _check_rows(num_cached, last_tokens, bucket, self.t_max)
+            _fill_inputs(self._graphs[bucket].buf, block_tables, num_cached, last_tokens, self.block_size)
         else:
-            self._copy_inputs(self._graphs[bucket].buf, inp)
+            inp = build_decode_static_inputs(
+                block_tables, num_cached, last_tokens, bucket, self.t_max, self.block_size,
+                self.device, self.dtype,
+            )
+            if bucket in self._graphs:
+                self._copy_inputs(self._graphs[bucket].buf, inp)
+            else:
+                self._capture(bucket, inp)
         self._graphs[bucket].graph.replay()
         return self._graphs[bucket].out[:b]
 

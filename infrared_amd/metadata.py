@@ -24,7 +24,8 @@ from collections.abc import Sequence
 import numpy as np
 import torch
 
-from infrared_amd.paged_kv_cache import PagedContext, PagedKVPool, row_split
+from infrared_amd._lib import check, lib, ptr, stream_ptr
+from infrared_amd.paged_kv_cache import PagedContext, PagedKVPool, row_split, to_device
 
 
 def slot(block_table: Sequence[int], pos: int, block_size: int) -> int:
@@ -45,13 +46,20 @@ def block_tables_tensor(
     copy per row, not per block id) and moved to the device at once."""
     lens = [len(r) for r in block_tables]
     w = max(lens, default=0) if width is None else width
-    if any(n > w for n in lens):
-        raise ValueError(f"a block table is longer than width {w}")
     arr = np.zeros((len(lens), w), dtype=np.int32)
-    for i, (r, n) in enumerate(zip(block_tables, lens)):
+    fill_tables(arr, block_tables)
+    return torch.from_numpy(arr).to(device)
+
+
+def fill_tables(arr: np.ndarray, block_tables: Sequence[Sequence[int]]) -> None:
+    """Copies each table into its row of ``arr`` (zeros past a table's end)."""
+    w = arr.shape[1]
+    for i, r in enumerate(block_tables):
+        n = len(r)
+        if n > w:
+            raise ValueError(f"a block table is longer than width {w}")
         if n:
             arr[i, :n] = r
-    return torch.from_numpy(arr).to(device)
 
 
 def packed_write_slots(
@@ -160,22 +168,22 @@ def prefill_context(
     lengths = [c + n for c, n in zip(num_cached, q_lens)]
     width = max(blocks_for(n, bs) for n in lengths) if lengths else 0
     rows = [r[: max(width, 1)] for r in block_tables]
-    bt = block_tables_tensor(rows, dev, width)
-    meta = torch.tensor([list(num_cached), list(q_lens)], dtype=torch.int32).to(dev)  # one host->device copy
-    nc_t, ql_t = meta[0], meta[1]
-    cu = torch.zeros(len(q_lens) + 1, dtype=torch.int32, device=dev)
-    cu[1:] = torch.cumsum(ql_t, 0)
-    ctx = PagedContext(
-        pool,
-        packed_write_slots(bt, nc_t, ql_t, bs),
-        None,
-        use_triton,
-        bt,
-        None,
-        cu,
-        nc_t.contiguous(),
-        max(q_lens, default=0),
-    )
+    total, n = sum(q_lens), len(q_lens)
+    if min(q_lens, default=0) < 0:
+        raise ValueError("q_lens must not be negative")
+    # one host array, one copy: tables, cached lengths, chunk starts
+    host = np.zeros(n * width + 2 * n + 1, dtype=np.int32)
+    fill_tables(host[: n * width].reshape(n, width), rows)
+    host[n * width : n * width + n] = num_cached
+    np.cumsum(np.asarray(q_lens, dtype=np.int64), out=host[n * width + n + 1 :])
+    flat = to_device(host, dev)
+    bt = flat[: n * width].view(n, width)
+    nc, cu = flat[n * width : n * width + n], flat[n * width + n :]
+    write_slots = torch.empty(total, dtype=torch.int64, device=flat.device)
+    check(lib().ir_packed_write_slots(
+        ptr(bt), width, width, ptr(nc), ptr(cu), n, total, bs, ptr(write_slots), stream_ptr(flat.device),
+    ), "ir_packed_write_slots")
+    ctx = PagedContext(pool, write_slots, None, use_triton, bt, None, cu, nc, max(q_lens, default=0))
     ctx.row_split = row_split(bt, num_cached, q_lens)
     if not with_mask:
         return ctx, None

@@ -412,22 +412,38 @@ def row_split(bt: torch.Tensor, num_cached: Sequence[int], q_lens: Sequence[int]
     dec_range = (first, first + nd)
     total = sum(q_lens)
     pre_range = (nd, total) if first == 0 else (0, first)
-    pre_cu = np.concatenate([[0], np.cumsum([q_lens[i] for i in pre], dtype=np.int64)])
-    host = torch.from_numpy(np.concatenate([
-        np.asarray(dec, np.int64), np.asarray(pre, np.int64), np.asarray([num_cached[i] + 1 for i in dec], np.int64),
-        pre_cu, np.asarray([num_cached[i] for i in pre], np.int64)]).astype(np.int64))
-    t = host.to(bt.device)  # one host->device copy
-    dec_idx, pre_idx, dec_ctx, pre_cu_t, pre_qs = torch.split(t, [nd, len(pre), nd, len(pre) + 1, len(pre)])
+    np_ = len(pre)
+    host = np.zeros(nd + 2 * np_ + 1, dtype=np.int32)  # one host->device copy
+    host[:nd] = [num_cached[i] + 1 for i in dec]
+    host[nd : nd + np_] = [num_cached[i] for i in pre]
+    np.cumsum(np.asarray([q_lens[i] for i in pre], dtype=np.int64), out=host[nd + np_ + 1 :])
+    t = to_device(host, bt.device)
+
+    def tables(ids):  # a run of rows is a view
+        if not ids or ids[-1] - ids[0] + 1 == len(ids):
+            return bt[ids[0] : ids[-1] + 1] if ids else bt[:0]
+        return bt[torch.tensor(ids, device=bt.device)]
+
     return RowSplit(
         dec_range=dec_range,
-        dec_tables=bt.index_select(0, dec_idx).contiguous(),
-        dec_ctx=dec_ctx.to(torch.int32),
+        dec_tables=tables(dec),
+        dec_ctx=t[:nd],
         pre_range=pre_range,
-        pre_tables=bt.index_select(0, pre_idx).contiguous(),
-        pre_cu=pre_cu_t.to(torch.int32),
-        pre_q_start=pre_qs.to(torch.int32),
+        pre_tables=tables(pre),
+        pre_cu=t[nd + np_ :],
+        pre_q_start=t[nd : nd + np_],
         pre_max_q=max((q_lens[i] for i in pre), default=0),
     )
+
+
+def to_device(host: np.ndarray, device: torch.device) -> torch.Tensor:
+    """A host array on ``device`` through pinned staging memory (torch's caching
+    allocator keeps it until the copy has run), so the host does not wait for
+    the stream as a copy from pageable memory does."""
+    t = torch.from_numpy(host)
+    if torch.device(device).type != "cuda":
+        return t.to(device)
+    return torch.empty(t.shape, dtype=t.dtype, pin_memory=True).copy_(t).to(device, non_blocking=True)
 
 
 @dataclass(slots=True)

@@ -847,3 +847,54 @@ def test_packed_step_runs_its_decode_rows_on_the_decode_kernels(order):
     ref = O.prefill_reference(q[0].cpu(), pool.k[0].cpu(), pool.v[0].cpu(), bt, paged.cu_seqlens_q.cpu(),
                               num_cached, bs, d**-0.5)
     assert (out[0].float().cpu() - ref).abs().max().item() <= 2e-2
+
+
+@pytest.mark.parametrize("b,bucket,t_max,bs,dtype", [
+    (1, 1, 1, 16, torch.float32), (3, 4, 255, 16, torch.bfloat16), (5, 8, 257, 32, torch.float16),
+    (2, 2, 4096, 8, torch.bfloat16), (4, 7, 100, 1, torch.float32),
+])
+def test_decode_inputs_kernel_matches_the_host_build(b, bucket, t_max, bs, dtype):
+    """The one-launch build of a decode step's inputs gives the elementwise build's
+    values: contexts from 1 token to t_max, short and over-long tables, padded rows."""
+    g = torch.Generator().manual_seed(t_max)
+    width = -(-t_max // bs)
+    cached = [0, t_max - 1, t_max // 2, min(bs, t_max - 1), t_max - 1][:b]
+    tables = [torch.randint(0, 999, (max(1, c // bs + 1) + (3 if i == 1 else 0),), generator=g).tolist()
+              for i, c in enumerate(cached)]
+    args = (tables, cached, [2**40 + i for i in range(b)], bucket, t_max, bs)
+    want = build_decode_static_inputs(*args, "cpu", dtype)
+    got = build_decode_static_inputs(*args, DEV, dtype)
+    assert width == got.block_tables.shape[1]
+    for name in type(want).__slots__:
+        w, x = getattr(want, name), getattr(got, name)
+        assert x.dtype == w.dtype and x.shape == w.shape and torch.equal(x.cpu(), w), name
+
+
+@pytest.mark.parametrize("num_cached,q_lens", [
+    ([0], [1]), ([0, 7, 33], [5, 0, 260]), ([15, 16, 17, 0], [1, 1, 1, 300]), ([3, 0, 40], [17, 31, 1]), ([5, 2], [0, 0]),
+    ([9, 4, 60, 8], [1, 0, 20, 40]),
+])
+def test_prefill_context_slots_match_the_per_token_slots(num_cached, q_lens):
+    """Write slots from the one-launch build, chunk starts and the row split's views,
+    empty chunks among them, against the per-token closed form."""
+    bs = 16
+    pool = PagedKVPool(1, 64, bs, 1, 64, torch.float32, device=DEV)
+    perm = torch.randperm(64, generator=torch.Generator().manual_seed(len(q_lens))).tolist()
+    tables, off = [], 0
+    for c, n in zip(num_cached, q_lens):
+        k = -(-(c + n) // bs)
+        tables.append(perm[off : off + k])
+        off += k
+    paged, _ = metadata.prefill_context(pool, tables, num_cached, q_lens)
+    want = [metadata.slot(t, c + j, bs) for t, c, n in zip(tables, num_cached, q_lens) for j in range(n)]
+    assert paged.write_slots.tolist() == want
+    assert paged.q_start.tolist() == num_cached
+    assert paged.cu_seqlens_q.tolist() == [sum(q_lens[:i]) for i in range(len(q_lens) + 1)]
+    s = paged.row_split
+    if s is not None:
+        dec, pre = [i for i, n in enumerate(q_lens) if n == 1], [i for i, n in enumerate(q_lens) if n > 1]
+        bt = paged.block_tables.tolist()
+        assert s.dec_tables.tolist() == [bt[i] for i in dec] and s.pre_tables.tolist() == [bt[i] for i in pre]
+        assert s.dec_ctx.tolist() == [num_cached[i] + 1 for i in dec]
+        assert s.pre_q_start.tolist() == [num_cached[i] for i in pre]
+        assert s.pre_cu.tolist() == [sum(q_lens[i] for i in pre[:j]) for j in range(len(pre) + 1)]
