@@ -159,6 +159,32 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
+_seam = None
+
+
+def seam():
+    """The native binding of the per-layer calls (``csrc/bind/seam.cpp``): they
+    take tensors, check them and make the C ABI call without leaving native
+    code."""
+    global _seam
+    if _seam is None:
+        lib()  # a library that was never built is reported as such
+        from infrared_amd import _seam as module
+
+        _seam = module
+    return _seam
+
+
+def stream_of(t: torch.Tensor) -> int:
+    """Raw handle of torch's current stream on ``t``'s device; raises for a
+    tensor that is not on a ROCm device."""
+    if not t.is_cuda:
+        require_device(t)
+    if _raw_stream is None:
+        return stream_ptr(t.device)
+    return _raw_stream(t.get_device())
+
+
 def check(rc: int, what: str) -> None:
     """Raises ``RuntimeError`` with the library's message when ``rc`` is an error."""
     if rc != 0:

@@ -3,7 +3,8 @@
 Run ``python -m infrared_amd.build`` (or ``__graft_entry__.build()``). Every
 ``csrc/*.hip`` / ``csrc/*.cpp`` file compiles to an object under ``_build/``
 in parallel, then one shared library is linked next to this file, where the
-loader in ``infrared_amd._lib`` looks for it.
+loader in ``infrared_amd._lib`` looks for it, and the Python binding
+(``csrc/bind``, host code against torch's headers) against that library.
 """
 
 from __future__ import annotations
@@ -14,6 +15,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(PKG_DIR)
@@ -22,6 +24,7 @@ INCLUDE = os.path.join(ROOT, "include")
 BUILD_DIR = os.path.join(PKG_DIR, "_build")
 LIB_NAME = "libinfrared_amd.so"
 LIB_PATH = os.path.join(PKG_DIR, LIB_NAME)
+SEAM_PATH = os.path.join(PKG_DIR, "_seam.so")  # the Python binding of the per-layer calls
 ARCH = "gfx950"
 
 # -packed-fp32-ops: no v_pk_{add,mul,fma}_f32 in device code (fp32 math is
@@ -82,19 +85,48 @@ def _compile(src: str, extra: list[str]) -> str:
     return obj
 
 
+def _build_seam(obj: str) -> None:
+    """Links the binding against the library next to it and torch (host code only)."""
+    from torch.utils import cpp_extension
+
+    libs = [f"-L{d}" for d in cpp_extension.library_paths()]
+    cmd = ["g++", "-shared", obj, "-o", SEAM_PATH + ".tmp", f"-L{PKG_DIR}", f"-l:{LIB_NAME}", "-Wl,-rpath,$ORIGIN",
+           *libs, "-ltorch", "-ltorch_cpu", "-lc10", "-ltorch_python"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"link of the binding failed:\n{res.stdout}{res.stderr}")
+    os.replace(SEAM_PATH + ".tmp", SEAM_PATH)
+
+
+def _compile_seam() -> str:
+    from torch.utils import cpp_extension
+
+    obj = os.path.join(BUILD_DIR, "seam.o")
+    incs = [f"-I{d}" for d in [INCLUDE, sysconfig.get_paths()["include"], *cpp_extension.include_paths()]]
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", *incs, "-c",
+           os.path.join(CSRC, "bind", "seam.cpp"), "-o", obj]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"compile of the binding failed:\n{res.stdout}{res.stderr}")
+    return obj
+
+
 def build(verbose: bool = False, extra_flags: list[str] | None = None) -> str:
     """Compiles every source and links the shared library; returns its path."""
     os.makedirs(BUILD_DIR, exist_ok=True)
     extra = list(extra_flags or [])
     srcs = sources()
-    with cf.ThreadPoolExecutor(max_workers=min(8, len(srcs))) as ex:
+    with cf.ThreadPoolExecutor(max_workers=min(8, len(srcs) + 1)) as ex:
+        seam = ex.submit(_compile_seam)
         objs = list(ex.map(lambda s: _compile(s, extra), srcs))
+        seam_obj = seam.result()
     tmp = LIB_PATH + ".tmp"
     cmd = [hipcc(), "-shared", "-fPIC", f"--offload-arch={ARCH}", *objs, "-o", tmp]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError(f"link failed:\n{res.stdout}{res.stderr}")
     os.replace(tmp, LIB_PATH)
+    _build_seam(seam_obj)
     if verbose:
         print(f"built {LIB_PATH} from {len(srcs)} sources")
     return LIB_PATH

@@ -13,7 +13,7 @@ from dataclasses import dataclass
 
 import torch
 
-from infrared_amd._lib import check, dtype_code, lib, ptr, require_device, stream_ptr
+from infrared_amd._lib import check, dtype_code, lib, ptr, require_device, seam, stream_of, stream_ptr
 
 
 def _last_dim_contiguous(name: str, t: torch.Tensor) -> None:
@@ -40,29 +40,7 @@ def kv_scatter(
     ``k``/``v``: ``[N, H_kv, D]``; ``slots``: ``[N]`` int64. Negative slots are
     skipped (padding sentinel); slots ``>= num_slots`` are skipped and flagged.
     """
-    dev = require_device(k_cache, v_cache, k, v, slots)
-    _cache_layer("kv_scatter", k_cache)
-    if v_cache.shape != k_cache.shape or v_cache.stride() != k_cache.stride():
-        raise RuntimeError("kv_scatter: k_cache and v_cache must have the same shape and strides")
-    n, h, d = k.shape
-    if v.shape != k.shape or (h, d) != tuple(k_cache.shape[1:]):
-        raise RuntimeError(
-            f"kv_scatter: k {tuple(k.shape)} / v {tuple(v.shape)} do not match pool rows "
-            f"{tuple(k_cache.shape[1:])}"
-        )
-    if k.dtype != k_cache.dtype or v.dtype != k_cache.dtype:
-        raise RuntimeError(f"kv_scatter: dtype mismatch ({k.dtype}, {v.dtype} vs pool {k_cache.dtype})")
-    if slots.dtype != torch.int64 or slots.shape != (n,):
-        raise RuntimeError(f"kv_scatter: slots must be int64 [{n}], got {slots.dtype} {tuple(slots.shape)}")
-    _last_dim_contiguous("kv_scatter k", k)
-    _last_dim_contiguous("kv_scatter v", v)
-    slots = slots.contiguous()
-    rc = lib().ir_kv_scatter(
-        ptr(k), k.stride(0), k.stride(1), ptr(v), v.stride(0), v.stride(1),
-        ptr(k_cache), ptr(v_cache), k_cache.stride(0), k_cache.stride(1), k_cache.shape[0],
-        ptr(slots), n, h, d, dtype_code(k_cache.dtype), ptr(err_flags), stream_ptr(dev),
-    )
-    check(rc, "ir_kv_scatter")
+    seam().kv_scatter(k_cache, v_cache, k, v, slots, err_flags, stream_of(k_cache))
 
 
 def gather_slots(
@@ -130,22 +108,14 @@ def decode_workspace_bytes(
     num_seqs: int, num_q_heads: int, num_kv_heads: int, head_dim: int, max_blocks: int,
     block_size: int, partition_tokens: int = 0,
 ) -> int:
-    return int(lib().ir_paged_decode_workspace_size(
+    return int(seam().decode_workspace_size(
         num_seqs, num_q_heads, num_kv_heads, head_dim, max_blocks, block_size, partition_tokens
     ))
 
 
 def decode_num_counters(num_seqs: int, num_q_heads: int, num_kv_heads: int) -> int:
     """int32 arrival counters a split decode needs (zero at rest; one buffer serves every shape)."""
-    return int(lib().ir_paged_decode_num_counters(num_seqs, num_q_heads, num_kv_heads))
-
-
-def _counters_for(counters: torch.Tensor | None, n: int, dev) -> torch.Tensor:
-    if counters is None:
-        return torch.zeros(max(n, 1), dtype=torch.int32, device=dev)
-    if counters.dtype != torch.int32 or not counters.is_contiguous() or counters.numel() < n:
-        raise RuntimeError(f"decode counters must be a contiguous int32 tensor of >= {n} zeros")
-    return counters
+    return int(seam().decode_num_counters(num_seqs, num_q_heads, num_kv_heads))
 
 
 def default_partition(num_seqs: int, num_kv_heads: int, max_blocks: int, block_size: int) -> int:
@@ -174,40 +144,8 @@ def paged_decode(
     when not given and the longest possible context needs more than one
     partition.
     """
-    dev = require_device(q, k_cache, v_cache, block_tables, context_lens)
-    _cache_layer("paged_decode", k_cache)
-    _check_tables("paged_decode", block_tables, context_lens)
-    if q.dim() != 3:
-        raise RuntimeError(f"paged_decode: q must be [B, H_q, D], got {tuple(q.shape)}")
-    b, hq, d = q.shape
-    h_kv = k_cache.shape[1]
-    if d != k_cache.shape[2] or q.dtype != k_cache.dtype or v_cache.shape != k_cache.shape:
-        raise RuntimeError("paged_decode: q / pool shape or dtype mismatch")
-    if block_tables.shape[0] != b:
-        raise RuntimeError("paged_decode: block_tables rows != batch")
-    _last_dim_contiguous("paged_decode q", q)
-    if out is None:
-        out = torch.empty(b, hq, d, dtype=q.dtype, device=dev)
-    max_blocks = block_tables.shape[1]
-    if partition_tokens <= 0:
-        partition_tokens = default_partition(b, h_kv, max_blocks, block_size)
-    need = decode_workspace_bytes(b, hq, h_kv, d, max_blocks, block_size, partition_tokens)
-    n_ctr = 0
-    if need > 0:
-        if workspace is None or workspace.numel() < need:
-            workspace = torch.empty(need, dtype=torch.uint8, device=dev)
-        n_ctr = decode_num_counters(b, hq, h_kv)
-        counters = _counters_for(counters, n_ctr, dev)
-    rc = lib().ir_paged_decode(
-        ptr(q), q.stride(0), q.stride(1), ptr(k_cache), ptr(v_cache), k_cache.stride(0),
-        k_cache.stride(1), k_cache.shape[0] // block_size, block_size, ptr(block_tables),
-        block_tables.stride(0), max_blocks, ptr(context_lens), ptr(out), out.stride(0),
-        out.stride(1), b, hq, h_kv, d, float(scale), dtype_code(q.dtype), partition_tokens,
-        ptr(counters) if need > 0 else None, n_ctr, ptr(workspace) if need > 0 else None, need,
-        ptr(err_flags), stream_ptr(dev),
-    )
-    check(rc, "ir_paged_decode")
-    return out
+    return seam().paged_decode(q, k_cache, v_cache, block_tables, context_lens, block_size, scale, out,
+                               partition_tokens, workspace, err_flags, counters, stream_of(q))
 
 
 @dataclass(frozen=True)
@@ -232,10 +170,16 @@ class DecodePlan:
     dtype: torch.dtype
     share_groups: bool = False
 
+    def native(self) -> tuple:
+        """The plan as the native decode call takes it."""
+        return (self.buf, (self.num_seqs, self.num_q_heads, self.num_kv_heads, self.max_blocks, self.block_size,
+                           self.num_blocks, self.slot_stride, self.head_stride),
+                self.dtype, PLAN_SHARE_GROUPS if self.share_groups else 0)
+
 
 def decode_plan_bytes(num_seqs: int, num_q_heads: int, num_kv_heads: int, max_blocks: int, block_size: int) -> int:
     """Plan bytes for this shape; 0 when it is not plannable (then use :func:`paged_decode`)."""
-    return int(lib().ir_paged_decode_plan_bytes(num_seqs, num_q_heads, num_kv_heads, max_blocks, block_size))
+    return int(seam().decode_plan_bytes(num_seqs, num_q_heads, num_kv_heads, max_blocks, block_size))
 
 
 _CU_COUNT: dict[int, int] = {}
@@ -266,7 +210,7 @@ def decode_plan_pays(num_seqs: int, num_q_heads: int, num_kv_heads: int, max_blo
 
 
 def planned_workspace_bytes(num_seqs: int, num_q_heads: int, num_kv_heads: int, head_dim: int) -> int:
-    return int(lib().ir_paged_decode_planned_workspace_bytes(num_seqs, num_q_heads, num_kv_heads, head_dim))
+    return int(seam().planned_workspace_bytes(num_seqs, num_q_heads, num_kv_heads, head_dim))
 
 
 def decode_plan(
@@ -323,37 +267,8 @@ def paged_decode_planned(
     """:func:`paged_decode` over a plan: ``q`` ``[B, H_q, D]`` -> ``[B, H_q, D]``.
     ``workspace`` (uint8 scratch) and ``counters`` (int32 zeros, left at zero)
     are allocated when not given."""
-    dev = require_device(q, k_cache, v_cache, plan.buf)
-    _cache_layer("paged_decode_planned", k_cache)
-    if q.dim() != 3:
-        raise RuntimeError(f"paged_decode_planned: q must be [B, H_q, D], got {tuple(q.shape)}")
-    b, hq, d = q.shape
-    if (b, hq) != (plan.num_seqs, plan.num_q_heads) or k_cache.shape[1] != plan.num_kv_heads:
-        raise RuntimeError("paged_decode_planned: q / pool heads differ from the plan's")
-    if (k_cache.shape[0] // plan.block_size != plan.num_blocks or k_cache.stride(0) != plan.slot_stride
-            or k_cache.stride(1) != plan.head_stride or k_cache.dtype != plan.dtype):
-        raise RuntimeError("paged_decode_planned: pool layout differs from the plan's")
-    if v_cache.shape != k_cache.shape or v_cache.stride() != k_cache.stride():
-        raise RuntimeError("paged_decode_planned: v_cache must match k_cache's shape and strides")
-    if d != k_cache.shape[2] or q.dtype != k_cache.dtype:
-        raise RuntimeError("paged_decode_planned: q / pool shape or dtype mismatch")
-    _last_dim_contiguous("paged_decode_planned q", q)
-    if out is None:
-        out = torch.empty(b, hq, d, dtype=q.dtype, device=dev)
-    need = planned_workspace_bytes(b, hq, plan.num_kv_heads, d)
-    if workspace is None or workspace.numel() < need:
-        workspace = torch.empty(need, dtype=torch.uint8, device=dev)
-    n_ctr = decode_num_counters(b, hq, plan.num_kv_heads)
-    counters = _counters_for(counters, n_ctr, dev)
-    rc = lib().ir_paged_decode_planned(
-        ptr(q), q.stride(0), q.stride(1), ptr(k_cache), ptr(v_cache), k_cache.stride(0), ptr(out),
-        out.stride(0), out.stride(1), b, hq, plan.num_kv_heads, d, plan.max_blocks, plan.block_size,
-        float(scale), dtype_code(q.dtype), PLAN_SHARE_GROUPS if plan.share_groups else 0, ptr(plan.buf),
-        ptr(counters), n_ctr, ptr(workspace),
-        workspace.numel(), ptr(err_flags), stream_ptr(dev),
-    )
-    check(rc, "ir_paged_decode_planned")
-    return out
+    return seam().paged_decode_planned(q, k_cache, v_cache, *plan.native(), scale, out, workspace, err_flags, counters,
+                                       stream_of(q))
 
 
 def paged_attention_masked(
@@ -374,44 +289,8 @@ def paged_attention_masked(
     ``run_if``: an int32 device flag; the kernel then writes ``out`` only
     when the flag is nonzero (read on the device, so it works under capture).
     """
-    dev = require_device(q, k_cache, v_cache, gather_slots, mask)
-    _cache_layer("paged_attention_masked", k_cache)
-    if q.dim() != 4:
-        raise RuntimeError(f"paged_attention_masked: q must be [B, Sq, H_q, D], got {tuple(q.shape)}")
-    b, sq, hq, d = q.shape
-    h_kv = k_cache.shape[1]
-    if d != k_cache.shape[2] or q.dtype != k_cache.dtype:
-        raise RuntimeError("paged_attention_masked: q / pool shape or dtype mismatch")
-    if gather_slots.dtype != torch.int64 or gather_slots.dim() != 2 or gather_slots.shape[0] != b:
-        raise RuntimeError("paged_attention_masked: gather_slots must be int64 [B, T]")
-    t = gather_slots.shape[1]
-    if mask.dim() != 4 or mask.shape[1] != 1:
-        raise RuntimeError(f"paged_attention_masked: mask must be [B, 1, Sq, T], got {tuple(mask.shape)}")
-    m = mask.expand(b, 1, sq, t)
-    _last_dim_contiguous("paged_attention_masked q", q)
-    if out is None:
-        out = torch.empty(b, sq, hq, d, dtype=q.dtype, device=dev)
-    if run_if is not None:
-        require_device(q, run_if)
-        if run_if.dtype != torch.int32 or run_if.numel() < 1:
-            raise RuntimeError("paged_attention_masked: run_if must be an int32 device tensor")
-    ws = None
-    # (a call of up to 192 keys is never split; a gated one of few columns needs no workspace)
-    if t > 192 and (run_if is None or sq * (hq // h_kv) > 32):
-        need = lib().ir_paged_attention_masked_workspace_size(
-            b, sq, t, hq, h_kv, d, dtype_code(q.dtype), dtype_code(m.dtype), m.stride(3))
-        if need > 0:
-            ws = torch.empty(need, dtype=torch.uint8, device=dev)
-    rc = lib().ir_paged_attention_masked_ws(
-        ptr(q), q.stride(0), q.stride(1), q.stride(2), ptr(k_cache), ptr(v_cache),
-        k_cache.stride(0), k_cache.stride(1), k_cache.shape[0], ptr(gather_slots),
-        gather_slots.stride(0), gather_slots.stride(1), ptr(m), m.stride(0), m.stride(2),
-        m.stride(3), dtype_code(m.dtype), ptr(out), out.stride(0), out.stride(1), out.stride(2),
-        b, sq, t, hq, h_kv, d, float(scale), dtype_code(q.dtype), ptr(err_flags), ptr(run_if),
-        ptr(ws), 0 if ws is None else ws.numel(), stream_ptr(dev),
-    )
-    check(rc, "ir_paged_attention_masked")
-    return out
+    return seam().paged_attention_masked(q, k_cache, v_cache, gather_slots, mask, scale, out, err_flags, run_if,
+                                         stream_of(q))
 
 
 def rope_kv_scatter(
@@ -433,36 +312,7 @@ def rope_kv_scatter(
     ``cos``/``sin``: fp32 ``[N, D]`` (``RotaryEmbedding`` output flattened over batch
     and sequence). ``q_out`` may be ``q`` itself (in place).
     """
-    dev = require_device(q, k, v, cos, sin, k_cache, v_cache, slots)
-    _cache_layer("rope_kv_scatter", k_cache)
-    if q.dim() != 3 or k.dim() != 3 or v.shape != k.shape:
-        raise RuntimeError("rope_kv_scatter: q [N, H_q, D], k and v [N, H_kv, D] expected")
-    n, hq, d = q.shape
-    if k.shape[0] != n or k.shape[2] != d or k.shape[1:] != k_cache.shape[1:]:
-        raise RuntimeError("rope_kv_scatter: k/v rows do not match q or the pool")
-    if q.dtype != k.dtype or k.dtype != k_cache.dtype or v.dtype != k.dtype:
-        raise RuntimeError("rope_kv_scatter: dtype mismatch")
-    if v_cache.stride() != k_cache.stride():
-        raise RuntimeError("rope_kv_scatter: k_cache and v_cache must share strides")
-    for name, t in (("cos", cos), ("sin", sin)):
-        if t.dtype != torch.float32 or t.shape != (n, d) or t.stride(1) != 1:
-            raise RuntimeError(f"rope_kv_scatter: {name} must be fp32 [N, D] with unit column stride")
-    if cos.stride(0) != sin.stride(0):
-        raise RuntimeError("rope_kv_scatter: cos and sin must share strides")
-    if slots.dtype != torch.int64 or slots.shape != (n,):
-        raise RuntimeError("rope_kv_scatter: slots must be int64 [N]")
-    for name, t in (("q", q), ("k", k), ("v", v)):
-        _last_dim_contiguous(f"rope_kv_scatter {name}", t)
-    if q_out is None:
-        q_out = torch.empty_like(q)
-    rc = lib().ir_rope_kv_scatter(
-        ptr(q), q.stride(0), q.stride(1), ptr(q_out), q_out.stride(0), q_out.stride(1), ptr(k), k.stride(0),
-        k.stride(1), ptr(v), v.stride(0), v.stride(1), ptr(cos), ptr(sin), cos.stride(0), ptr(k_cache),
-        ptr(v_cache), k_cache.stride(0), k_cache.stride(1), k_cache.shape[0], ptr(slots.contiguous()), n, hq,
-        k.shape[1], d, dtype_code(q.dtype), ptr(err_flags), stream_ptr(dev),
-    )
-    check(rc, "ir_rope_kv_scatter")
-    return q_out
+    return seam().rope_kv_scatter(q, k, v, cos, sin, k_cache, v_cache, slots, q_out, err_flags, stream_of(q))
 
 
 PLAN_SHARE_GROUPS = 1  # IR_PLAN_SHARE_GROUPS
@@ -620,57 +470,19 @@ def paged_prefill(
     read from those rows (``ERR_WRITE_SLOT`` is flagged where a token's write
     slot is not its block-table slot).
     """
-    dev = require_device(q, k_cache, v_cache, block_tables, cu_seqlens_q, q_start)
-    _cache_layer("paged_prefill", k_cache)
-    if q.dim() != 3:
-        raise RuntimeError(f"paged_prefill: q must be [total_q, H_q, D], got {tuple(q.shape)}")
-    total_q, hq, d = q.shape
-    h_kv = k_cache.shape[1]
-    if d != k_cache.shape[2] or q.dtype != k_cache.dtype or v_cache.shape != k_cache.shape:
-        raise RuntimeError("paged_prefill: q / pool shape or dtype mismatch")
-    if v_cache.stride() != k_cache.stride():
-        raise RuntimeError("paged_prefill: k_cache and v_cache must share strides")
-    b = block_tables.shape[0]
-    if block_tables.dtype != torch.int32 or block_tables.dim() != 2 or block_tables.stride(1) != 1:
-        raise RuntimeError("paged_prefill: block_tables must be int32 [B, max_blocks] with unit column stride")
-    for name, t, n in (("cu_seqlens_q", cu_seqlens_q, b + 1), ("q_start", q_start, b)):
-        if t.dtype != torch.int32 or t.shape != (n,) or not t.is_contiguous():
-            raise RuntimeError(f"paged_prefill: {name} must be contiguous int32 [{n}]")
-    _last_dim_contiguous("paged_prefill q", q)
+    stream = stream_of(q)
     if plan is not None:
-        require_device(q, plan.buf)
+        hq, d = q.shape[-2:]
         if (plan.num_seqs, plan.max_q_len, plan.num_q_heads, plan.num_kv_heads, plan.head_dim) != (
-                b, int(max_q_len), hq, h_kv, d):
+                block_tables.shape[0], int(max_q_len), hq, k_cache.shape[1], d):
             raise RuntimeError("paged_prefill: the plan was built for other shapes")
         if plan.f32 != (q.dtype == torch.float32):
             raise RuntimeError("paged_prefill: the plan was built for "
                                + ("fp32" if plan.f32 else "16-bit") + f" calls, q is {q.dtype}")
-    if out is None:
-        out = torch.empty(total_q, hq, d, dtype=q.dtype, device=dev)
-    kn = vn = slots = None
-    n_write = 0
-    if new_kv is not None:
-        kn, vn, slots = new_kv
-        require_device(q, kn, vn, slots)
-        n_write = kn.shape[0]
-        if (kn.shape != (n_write, h_kv, d) or vn.shape != kn.shape or kn.dtype != q.dtype or vn.dtype != q.dtype
-                or slots.dtype != torch.int64 or slots.shape != (n_write,)):
-            raise RuntimeError("paged_prefill: new_kv must be (k, v [N, H_kv, D] of q's dtype, slots int64 [N])")
-        _last_dim_contiguous("paged_prefill new k", kn)
-        _last_dim_contiguous("paged_prefill new v", vn)
-        slots = slots.contiguous()
-    rc = lib().ir_paged_prefill(
-        ptr(q), q.stride(0), q.stride(1), ptr(k_cache), ptr(v_cache), k_cache.stride(0), k_cache.stride(1),
-        k_cache.shape[0] // block_size, block_size, ptr(block_tables), block_tables.stride(0),
-        block_tables.shape[1], ptr(cu_seqlens_q), ptr(q_start), b, total_q, int(max_q_len), ptr(out),
-        out.stride(0), out.stride(1), hq, h_kv, d, float(scale), dtype_code(q.dtype),
-        None if plan is None else ptr(plan.buf), 0 if plan is None else plan.buf.numel(),
-        ptr(kn), 0 if kn is None else kn.stride(0), 0 if kn is None else kn.stride(1),
-        ptr(vn), 0 if vn is None else vn.stride(0), 0 if vn is None else vn.stride(1),
-        ptr(slots), n_write, int(src_row0), ptr(err_flags), stream_ptr(dev),
-    )
-    check(rc, "ir_paged_prefill")
-    return out
+    kn, vn, slots = (None, None, None) if new_kv is None else new_kv
+    return seam().paged_prefill(q, k_cache, v_cache, block_tables, cu_seqlens_q, q_start, int(max_q_len), block_size,
+                                scale, out, err_flags, None if plan is None else plan.buf, kn, vn, slots,
+                                int(src_row0), stream)
 
 
 FORM_CLEAR_ON_FAIL = 1  # IR_FORM_CLEAR_ON_FAIL

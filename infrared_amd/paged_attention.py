@@ -51,6 +51,8 @@ from __future__ import annotations
 import torch
 
 from infrared_amd import kernels
+from infrared_amd._lib import seam, stream_of
+from infrared_amd.paged_kv_cache import PagedKVPool
 
 
 def paged_attention(
@@ -78,8 +80,7 @@ def paged_attention(
         raise RuntimeError(
             f"paged_attention: q {tuple(q.shape)} inconsistent with k {tuple(k.shape)} and n_rep={n_rep}"
         )
-    return _attend(q, paged, mask, layer_idx, scale,
-                   new_kv=(k.reshape(-1, h_kv, d), v.reshape(-1, h_kv, d), paged.write_slots))
+    return _attend(q, paged, mask, layer_idx, scale, new_kv=(k, v, paged.write_slots))
 
 
 def rope_paged_attention(
@@ -119,18 +120,33 @@ def rope_paged_attention(
 
 def _attend(q: torch.Tensor, paged, mask: torch.Tensor | None, layer_idx: int, scale: float,
             new_kv: tuple | None = None) -> torch.Tensor:
-    """Attention over the pool. ``new_kv`` = (k rows, v rows, write slots) of
-    this step, not yet written: the chunked-prefill paths fold the write into
-    their launch, every other path writes them first (``pool.write``)."""
+    """Attention over the pool. ``new_kv`` = (k, v ``[B, Sq, H_kv, D]``, write
+    slots) of this step, not yet written: the chunked-prefill paths fold the
+    write into their launch, every other path writes them first (as
+    ``pool.write``)."""
     pool = paged.pool
     b, sq = q.shape[:2]
     k_layer, v_layer = pool.k[layer_idx], pool.v[layer_idx]
     err = getattr(pool, "err_flags", None)
-    fusable = new_kv is not None and _fusable(pool, layer_idx, new_kv)
 
     def write():
-        if new_kv is not None:
-            pool.write(layer_idx, *new_kv)
+        if new_kv is None:
+            return
+        k, v, slots = new_kv
+        if k.dim() != 4 or v.dim() != 4 or getattr(type(pool), "write", None) is not PagedKVPool.write or pool.strict:
+            h_kv, d = k.shape[-2:]
+            pool.write(layer_idx, k.reshape(-1, h_kv, d), v.reshape(-1, h_kv, d), slots)
+        else:  # PagedKVPool.write on the layer already at hand
+            seam().write_step(k_layer, v_layer, k, v, slots, err, stream_of(k_layer))
+
+    def rows():
+        """``new_kv`` as rows ``[N, H_kv, D]`` if the prefill launch can take the write, else None."""
+        if new_kv is None:
+            return None
+        k, v, slots = new_kv
+        h_kv, d = k.shape[-2:]
+        r = (k.reshape(-1, h_kv, d), v.reshape(-1, h_kv, d), slots)
+        return r if _fusable(pool, layer_idx, r) else None
 
     block_tables = getattr(paged, "block_tables", None)
     context_lens = getattr(paged, "context_lens", None)
@@ -144,14 +160,15 @@ def _attend(q: torch.Tensor, paged, mask: torch.Tensor | None, layer_idx: int, s
         and q.dtype in (torch.bfloat16, torch.float16, torch.float32)
     ):
         split = getattr(paged, "row_split", None)
-        if not fusable:
+        fused = rows()
+        if fused is None:
             write()
         if split is not None:
-            out = _split_step(q, pool, layer_idx, split, scale, err, new_kv if fusable else None)
+            out = _split_step(q, pool, layer_idx, split, scale, err, fused)
         else:
             max_q = getattr(paged, "max_q_len", 0) or b * sq
             out = _prefill(q, pool, layer_idx, block_tables, cu_seqlens_q, q_start, max_q, paged, scale, err,
-                           new_kv=new_kv if fusable else None)
+                           new_kv=fused)
     elif paged.use_triton and block_tables is not None and context_lens is not None and sq == 1:
         write()
         out = _decode(q, pool, layer_idx, block_tables, context_lens, paged, scale, err)
@@ -174,9 +191,9 @@ def _attend(q: torch.Tensor, paged, mask: torch.Tensor | None, layer_idx: int, s
             # the reference's packed prefill / mixed-step frame: when it has
             # that form, run the chunked-prefill kernel over derived metadata
             vform = pool.reference_varlen_form(paged.gather_slots, mask)
-        if vform is None or not fusable:
+        fused = rows() if vform is not None else None
+        if fused is None:
             write()
-            fusable = False
         verdict = form.verdict() if form is not None else None
         if form is not None and verdict is False:
             # the check's published verdict: not the decode form
@@ -195,10 +212,10 @@ def _attend(q: torch.Tensor, paged, mask: torch.Tensor | None, layer_idx: int, s
                     run_if=form.gate if verdict is None else None,
                 )
         elif vform is not None and vform.row_split is not None:
-            out = _split_step(q, pool, layer_idx, vform.row_split, scale, err, new_kv if fusable else None)
+            out = _split_step(q, pool, layer_idx, vform.row_split, scale, err, fused)
         elif vform is not None:
             out = _prefill(q, pool, layer_idx, vform.block_tables, vform.cu_seqlens_q, vform.q_start,
-                           vform.max_q_len, vform, scale, err, new_kv=new_kv if fusable else None)
+                           vform.max_q_len, vform, scale, err, new_kv=fused)
         else:
             out = kernels.paged_attention_masked(
                 q, k_layer, v_layer, paged.gather_slots, mask, scale, err_flags=err
@@ -315,9 +332,7 @@ def _decode(q, pool, layer_idx: int, block_tables, context_lens, holder, scale: 
         ctr = pool.decode_counters(kernels.decode_num_counters(b, hq, h_kv))
         if own:
             _hold(holder, ws, ctr)
-        out = kernels.paged_decode_planned(
-            q.reshape(b, hq, d), k_layer, v_layer, plan, scale, out=out, workspace=ws, err_flags=err, counters=ctr
-        )
+        return seam().decode_step_planned(q, k_layer, v_layer, *plan.native(), scale, out, ws, err, ctr, stream_of(q))
     else:
         ws = ctr = None
         if hasattr(pool, "workspace"):
@@ -327,12 +342,8 @@ def _decode(q, pool, layer_idx: int, block_tables, context_lens, holder, scale: 
                 ctr = pool.decode_counters(kernels.decode_num_counters(b, hq, h_kv))
         if ws is not None and getattr(holder, "gate", None) is not None:
             _hold(holder, ws, ctr)
-        out = kernels.paged_decode(
-            q.reshape(b, hq, d), k_layer, v_layer, block_tables, context_lens,
-            pool.block_size, scale, out=out, workspace=ws, err_flags=err, counters=ctr,
-        )
-    return out.view(b, 1, hq, d)
-
+        return seam().decode_step(q, k_layer, v_layer, block_tables, context_lens, pool.block_size, scale, out, ws, err,
+                                  ctr, stream_of(q))
 
 
 def _hold(holder, *tensors: torch.Tensor) -> None:
