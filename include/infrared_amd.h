@@ -316,9 +316,11 @@ int ir_paged_attention_masked(const void* q, int64_t q_b_stride, int64_t q_s_str
  * ir_paged_attention_masked that may cut the keys of a call with too few
  * workgroups for the device into parts, their fp32 partial rows in `workspace`
  * (16-byte aligned scratch, nothing kept in it between calls; null: one part).
- * It uses as many parts as pay and `workspace_bytes` holds;
- * ir_paged_attention_masked_workspace_size gives the bytes for all of them (0:
- * one part is best), at most 256 MiB.
+ * It uses as many parts as pay and `workspace_bytes` holds. With a workspace, a
+ * long frame's mask and keys are first surveyed for the key tiles that add exactly
+ * nothing to a block of query rows, which are then left out.
+ * ir_paged_attention_masked_workspace_size gives the bytes for all of this (0:
+ * nothing would be used), at most 256 MiB of parts and the survey's few MB.
  */
 int64_t ir_paged_attention_masked_workspace_size(int batch, int seq_q, int seq_k,
                                                  int num_q_heads, int num_kv_heads,

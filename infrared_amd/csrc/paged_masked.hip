@@ -51,6 +51,11 @@ struct MaskedArgs {
   int serial;  // the workgroup takes every part itself, one after the other
   float* ws_o;
   float* ws_ml;
+  // survey of the mask and the keys (vis null: none), see paged_masked_survey_kernel
+  uint8_t* vis;      // [batch][128-column block][tile, padded to 64]: any key visible
+  uint8_t* tok_vis;  // [batch][128-column block][group of 8 tiles][32 tokens]: a key clearly visible
+  int2* walks;       // [batch][KV head][128-column block]: (parts, tiles) of its walk, parts < 0: of all tiles
+  float* bounds;     // [batch][KV head][tile]: largest |K|, inf if K or V is not finite or a slot is bad
 };
 
 // Bits of one mask element; mask_val converts them. Split so that a load can
@@ -253,6 +258,180 @@ void paged_masked_kernel(MaskedArgs a) {
   }
 }
 
+// ---------------------------------------------------------------- survey
+//
+// A packed frame's mask is block-diagonal: most of its 64-key tiles hold nothing
+// a 128-column block may see, and what they add is exactly zero -- provided every
+// row sees some key clearly, no score is large enough to bring a masked key back,
+// and V is finite (0 * inf is NaN). This kernel finds out, so that the wide
+// kernel may leave those tiles out with the same result bit by bit: per (KV head,
+// tile) the largest |K|, and per (column block, tile) whether any mask value is
+// above kMasked, with a flag for each token that has one above kClear. One pass
+// over the mask and the frame's keys. 610 tokens x 5333 keys (8 sequences),
+// 28/4 heads of 128, bf16: 9 us + 7.5 us for the walks, after which the wide kernel
+// takes 35 us instead of 109.
+constexpr float kMasked = -6e4f;    // fp16's finfo.min is -65504
+constexpr float kClear = -1e3f;
+constexpr float kScoreBound = 25e3f;  // 2 x this + kMasked - kClear stays far below any exponent
+constexpr int kSurveyTiles = 8;     // tiles of a mask workgroup: 8 keys a lane
+constexpr int kPartTiles = 6;       // tiles of a surveyed block worth a part of their own
+constexpr int kSurveyMin = 16;      // tiles from which a call is surveyed
+
+template <int DT, int D>
+__global__ __launch_bounds__(256) void paged_masked_survey_kernel(MaskedArgs a, int nt, int n_rtw) {
+  using E = Elem<DT>;
+  constexpr int PPR = D / 8;
+  __shared__ uint32_t red[4][kSurveyTiles];
+  if (a.run_if && *a.run_if == 0) return;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int n_key_wgs = a.batch * a.num_kv_heads * nt;
+  if ((int)blockIdx.x < n_key_wgs) {
+    // keys of one tile of one KV head
+    const int t = blockIdx.x % nt, kvh = blockIdx.x / nt % a.num_kv_heads, b = blockIdx.x / nt / a.num_kv_heads;
+    const uint16_t* kc = (const uint16_t*)a.kc + (int64_t)kvh * a.c_head;
+    const uint16_t* vc = (const uint16_t*)a.vc + (int64_t)kvh * a.c_head;
+    constexpr uint32_t kInfBits = DT == IR_DTYPE_BF16 ? 0x7f80u : 0x7c00u;
+    uint32_t big = 0;  // largest |element| of K as bits; the infinity's for what disallows a survey
+    bool bad = false;
+#pragma unroll
+    for (int i = 0; i < kTileKeys * PPR / 256; ++i) {
+      const int q = tid + 256 * i, key = t * kTileKeys + q / PPR;
+      if (key >= a.seq_k) continue;
+      const int64_t sl = a.gs[(int64_t)b * a.gs_b + (int64_t)key * a.gs_t];
+      if (sl < 0 || sl >= a.num_slots) {
+        bad = true;
+        big = kInfBits;
+        continue;
+      }
+      const int64_t off = sl * a.c_slot + (q % PPR) * 8;
+      const u32x4 k = *(const u32x4*)(kc + off), v = *(const u32x4*)(vc + off);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        big = max(big, max(k[e] & 0x7fffu, k[e] >> 16 & 0x7fffu));
+        if ((v[e] & 0x7fffu) >= kInfBits || (v[e] >> 16 & 0x7fffu) >= kInfBits) big = max(big, kInfBits);
+      }
+    }
+    if (bad) flag_error(a.err, IR_ERR_GATHER_RANGE);
+#pragma unroll
+    for (int o = 32; o; o >>= 1) big = max(big, (uint32_t)__shfl_xor((int)big, o));
+    if (lane == 0) red[w][0] = big;
+    __syncthreads();
+    if (tid == 0) {
+      big = max(max(red[0][0], red[1][0]), max(red[2][0], red[3][0]));
+      a.bounds[blockIdx.x] = big >= kInfBits ? __builtin_inff() : E::lo(big);
+    }
+    return;
+  }
+  // the mask of one column block's tokens over kSurveyTiles tiles: a wavefront
+  // per token, 8 keys a lane
+  const int n_groups = (nt + kSurveyTiles - 1) / kSurveyTiles;
+  const int idx = blockIdx.x - n_key_wgs;
+  const int grp = idx % n_groups, rt = idx / n_groups % n_rtw, b = idx / n_groups / n_rtw;
+  const int rows = a.seq_q * a.n_rep;
+  const int tok0 = rt * kWideCols / a.n_rep;
+  const int ntok = min(rt * kWideCols + kWideCols - 1, rows - 1) / a.n_rep - tok0 + 1;
+  const int k0 = grp * (kSurveyTiles * kTileKeys) + lane * 8;
+  uint8_t* tok_vis = a.tok_vis + (((int64_t)b * n_rtw + rt) * n_groups + grp) * 32;
+  bool any = false;
+  for (int tok = w; tok < ntok; tok += 4) {
+    const uint16_t* row = (const uint16_t*)a.mask + (int64_t)b * a.m_b + (int64_t)(tok0 + tok) * a.m_s;
+    bool clear = false;
+    if (k0 + 8 <= a.seq_k) {
+      uint32_t x[4];
+      __builtin_memcpy(x, row + k0, 16);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float lo = E::lo(x[e]), hi = E::hi(x[e]);
+        any |= !(lo <= kMasked) || !(hi <= kMasked);
+        clear |= lo > kClear || hi > kClear;
+      }
+    } else {
+      for (int t = k0; t < a.seq_k; ++t) {
+        const float v = E::lo(row[t]);
+        any |= !(v <= kMasked);
+        clear |= v > kClear;
+      }
+    }
+    const bool c = __any(clear);
+    if (lane == 0) tok_vis[tok] = c;
+  }
+  const uint64_t bits = __ballot(any);  // 8 lanes a tile
+  if (lane < kSurveyTiles) red[w][lane] = (bits >> (8 * lane) & 0xff) != 0;
+  __syncthreads();
+  if (tid < kSurveyTiles && grp * kSurveyTiles + tid < nt) {
+    const int ntp = (nt + 63) / 64 * 64;
+    a.vis[((int64_t)b * n_rtw + rt) * ntp + grp * kSurveyTiles + tid] =
+        (red[0][tid] | red[1][tid] | red[2][tid] | red[3][tid]) != 0;
+  }
+}
+
+// The walk of each column block: which tiles (those some token of it sees, or all
+// of them when the survey found a reason) and how many parts they are worth. A
+// kernel of its own so that the wide kernel's workgroups past a block's parts end
+// after one load.
+template <int DT, int D>
+__global__ __launch_bounds__(256) void paged_masked_walks_kernel(MaskedArgs a, int nt, int n_rtw) {
+  using E = Elem<DT>;
+  __shared__ float red[8];
+  __shared__ int cnt[4];
+  if (a.run_if && *a.run_if == 0) return;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int rt = blockIdx.x % n_rtw, kvh = blockIdx.x / n_rtw % a.num_kv_heads;
+  const int b = blockIdx.x / n_rtw / a.num_kv_heads;
+  const int rows = a.seq_q * a.n_rep, row0 = rt * kWideCols;
+  const int tok0 = row0 / a.n_rep;
+  const int ntok = min(row0 + kWideCols - 1, rows - 1) / a.n_rep - tok0 + 1;
+  float kmax = 0.f;
+  for (int t = tid; t < nt; t += 256) kmax = fmaxf(kmax, a.bounds[((int64_t)b * a.num_kv_heads + kvh) * nt + t]);
+  uint32_t qbig = 0;
+#pragma unroll
+  for (int i = 0; i < kWideCols * (D / 8) / 256; ++i) {
+    const int q = tid + 256 * i, row = row0 + q / (D / 8);
+    if (row >= rows) continue;
+    const int sq = row / a.n_rep, head = kvh * a.n_rep + row - sq * a.n_rep;
+    const u32x4 x = *(const u32x4*)((const uint16_t*)a.q + (int64_t)b * a.q_b + (int64_t)sq * a.q_s +
+                                    (int64_t)head * a.q_h + (q % (D / 8)) * 8);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) qbig = max(qbig, max(x[e] & 0x7fffu, x[e] >> 16 & 0x7fffu));
+  }
+  bool clear = true;  // a lane of wavefront 0 per token
+  if (tid < ntok) {
+    const int n_groups = (nt + kSurveyTiles - 1) / kSurveyTiles;
+    const uint8_t* tv = a.tok_vis + ((int64_t)b * n_rtw + rt) * n_groups * 32 + tid;
+    uint32_t any = 0;
+    for (int i = 0; i < n_groups; ++i) any |= tv[i * 32];
+    clear = any != 0;
+  }
+  const uint8_t* vis = a.vis + ((int64_t)b * n_rtw + rt) * ((nt + 63) / 64 * 64);
+  int n = 0;
+  for (int t = tid; t < nt; t += 256) n += vis[t] != 0;
+#pragma unroll
+  for (int o = 32; o; o >>= 1) {
+    kmax = fmaxf(kmax, __shfl_xor(kmax, o));
+    qbig = max(qbig, (uint32_t)__shfl_xor((int)qbig, o));
+    n += __shfl_xor(n, o);
+  }
+  if (!__all(clear)) kmax = __builtin_inff();
+  if (lane == 0) {
+    red[w] = kmax;
+    red[4 + w] = E::lo(qbig);
+    cnt[w] = n;
+  }
+  __syncthreads();
+  if (tid != 0) return;
+  const float km = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+  bool ok = true;  // (q: a NaN's bits are above the infinity's, and compare false below)
+  float qm = 0.f;
+  for (int i = 0; i < 4; ++i) {
+    ok = ok && red[4 + i] < __builtin_inff();
+    qm = fmaxf(qm, red[4 + i]);
+  }
+  ok = ok && km < __builtin_inff() && km * qm * (D * fabsf(a.scale)) < kScoreBound;
+  n = ok ? cnt[0] + cnt[1] + cnt[2] + cnt[3] : nt;
+  const int np = min(a.parts, max(1, (n + kPartTiles - 1) / kPartTiles));
+  a.walks[blockIdx.x] = make_int2(ok ? np : -np, n);
+}
+
 // ---------------------------------------------------------------- many columns, 16-bit
 //
 // Chunks: a workgroup of 4 wavefronts owns 128 columns of one KV head and one
@@ -293,16 +472,32 @@ void paged_masked_wide_kernel(MaskedArgs a) {
 
   const int tid = threadIdx.x;
   const int lane = tid & 63, w = tid >> 6, g = lane >> 4, c = lane & 15;
-  // workgroups that walk the same keys are a multiple of (KV heads x parts x
-  // sequences) apart, so they mostly share an XCD's L2
-  const int per_rt = a.num_kv_heads * a.parts * a.batch;
-  const int rt = blockIdx.x / per_rt;
-  int idx = blockIdx.x - rt * per_rt;
+  // parts outermost: the workgroups of a surveyed block's unused parts come last,
+  // and those in use spread evenly over the XCDs (innermost: 49 us instead of 35);
+  // with KV heads innermost the blocks that walk a KV head's keys share a few
+  // XCDs' L2s
+  const int n_rtw = (a.seq_q * a.n_rep + kWideCols - 1) / kWideCols;
+  int idx = blockIdx.x;
   const int kvh = idx % a.num_kv_heads;
   idx /= a.num_kv_heads;
-  const int part = idx % a.parts;
-  const int b = idx / a.parts;
+  const int rt = idx % n_rtw;
+  idx /= n_rtw;
+  const int b = idx % a.batch;
+  const int part = idx / a.batch;
   const int rows = a.seq_q * a.n_rep;
+  const int ntiles = (a.seq_k + BN - 1) / BN;
+  // the tiles and parts of this block's walk: the survey's, else all of them
+  int n = ntiles, np = a.parts;
+  const uint8_t* vis = nullptr;
+  if constexpr (ML) {
+    if (a.vis) {
+      const int2 x = a.walks[((int64_t)b * a.num_kv_heads + kvh) * n_rtw + rt];
+      np = abs(x.x);
+      if (part >= np) return;  // (the grid has parts for the longest walk)
+      n = x.y;
+      if (x.x > 0) vis = a.vis + ((int64_t)b * n_rtw + rt) * ((ntiles + 63) / 64 * 64);
+    }
+  }
 
   struct Col {
     int row, sq, head;
@@ -337,9 +532,36 @@ void paged_masked_wide_kernel(MaskedArgs a) {
   const uint16_t* kc = (const uint16_t*)a.kc + (int64_t)kvh * a.c_head;
   const uint16_t* vc = (const uint16_t*)a.vc + (int64_t)kvh * a.c_head;
   const int64_t* gs = a.gs + (int64_t)b * a.gs_b;
-  const int ntiles = (a.seq_k + BN - 1) / BN;
-  const int t_lo = (int)((int64_t)part * ntiles / a.parts);
-  const int t_hi = (int)((int64_t)(part + 1) * ntiles / a.parts);
+
+  // tiles to walk, 64 to a word; this part's share of them
+  auto word = [&](int wi) -> uint64_t {
+    const int t = wi * 64 + lane;
+    return __ballot(t < ntiles && (!vis || vis[t]));
+  };
+  int skip = (int)((int64_t)part * n / np);
+  int left = (int)((int64_t)(part + 1) * n / np) - skip;
+  int wi = 0;
+  uint64_t wbits = word(0);
+  while (skip > 0 && __popcll(wbits) <= skip) {  // whole words before the share
+    skip -= __popcll(wbits);
+    wbits = word(++wi);
+  }
+  for (; skip > 0; --skip) wbits &= wbits - 1;
+  // the share's next tile, or -1
+  auto next = [&]() {
+    if (left <= 0) return -1;
+    while (!wbits) {
+      if (++wi * 64 >= ntiles) {
+        left = 0;
+        return -1;
+      }
+      wbits = word(wi);
+    }
+    --left;
+    const int t = wi * 64 + __builtin_ctzll(wbits);
+    wbits &= wbits - 1;
+    return __builtin_amdgcn_readfirstlane(t);
+  };
 
   bool bad = false;
   u32x4 kreg[KPT], vreg[KPT];
@@ -349,13 +571,13 @@ void paged_masked_wide_kernel(MaskedArgs a) {
   int64_t s_raw = -1;
   auto load_slot = [&](int kb) {
     const int t = kb * BN + tid;
-    if (tid < BN) s_raw = t < a.seq_k ? gs[(int64_t)t * a.gs_t] : -1;
+    if (tid < BN) s_raw = kb >= 0 && t < a.seq_k ? gs[(int64_t)t * a.gs_t] : -1;
   };
-  auto hand_slot = [&](int kb) {
+  auto hand_slot = [&](int kb, int buf) {
     if (tid >= BN) return;
     const bool in = s_raw >= 0 && s_raw < a.num_slots;
-    bad |= !in && kb * BN + tid < a.seq_k;
-    slot_lds[kb & 1][tid] = in ? (int)s_raw : -1;
+    bad |= !in && kb >= 0 && kb * BN + tid < a.seq_k;
+    slot_lds[buf][tid] = in ? (int)s_raw : -1;
   };
   // mask pieces of tile kb (4 keys of one of the workgroup's tokens each); keys
   // past the end repeat the last one, their scores are -inf
@@ -378,12 +600,12 @@ void paged_masked_wide_kernel(MaskedArgs a) {
   };
   // K and V pieces of tile kb; unusable keys read slot 0 and are zeroed where
   // they are staged
-  auto issue = [&](int kb) {
+  auto issue = [&](int kb, int buf) {
     if constexpr (ML) load_mask(kb);
 #pragma unroll
     for (int i = 0; i < KPT; ++i) {
       const int q = tid + NT * i;
-      const int sl = slot_lds[kb & 1][q / PPR];
+      const int sl = slot_lds[buf][q / PPR];
       use[i] = sl >= 0;
       const int64_t off = (int64_t)(use[i] ? sl : 0) * a.c_slot + (q % PPR) * 8;
       kreg[i] = *(const u32x4*)(kc + off);
@@ -420,10 +642,10 @@ void paged_masked_wide_kernel(MaskedArgs a) {
     for (int dt = 0; dt < DTL; ++dt) acc[ct][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
 
-  auto tile = [&](int kb) {
+  auto tile = [&](int kb, int buf) {
     const int k0 = kb * BN;
-    const uint16_t* kl = ks_lds[kb & 1];
-    const uint16_t* vl = vs_lds[kb & 1];
+    const uint16_t* kl = ks_lds[buf];
+    const uint16_t* vl = vs_lds[buf];
     // the mask of keys k0 + 16 kt + 4 g .. + 3 of each column
     uint32_t mk[CT][4][MB];
     if constexpr (ML) {
@@ -471,7 +693,7 @@ void paged_masked_wide_kernel(MaskedArgs a) {
       for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
         for (int kt = 0; kt < 4; ++kt) {
-          const u32x2 x = *(const u32x2*)&mk_lds[kb & 1][mtok[ct] * MP + 16 * kt + 4 * g];
+          const u32x2 x = *(const u32x2*)&mk_lds[buf][mtok[ct] * MP + 16 * kt + 4 * g];
           mk[ct][kt][0] = x[0];
           mk[ct][kt][1] = x[1];
         }
@@ -490,7 +712,7 @@ void paged_masked_wide_kernel(MaskedArgs a) {
           sc[ct][kt][r] = fmaxf((sc[ct][kt][r] * a.scale + mv) * kLog2e, -__FLT_MAX__);
         }
     // keys that may not be read: rare, so one vote over the tile's 64 keys
-    const uint64_t okm = __ballot(key_ok[kb & 1][lane] != 0);
+    const uint64_t okm = __ballot(key_ok[buf][lane] != 0);
     if (okm != ~0ull) {
 #pragma unroll
       for (int kt = 0; kt < 4; ++kt)
@@ -547,27 +769,35 @@ void paged_masked_wide_kernel(MaskedArgs a) {
 
   if (a.num_slots <= 0) {
     bad = a.seq_k > 0;
-  } else if (t_lo < t_hi) {
-    load_slot(t_lo);
-    hand_slot(t_lo);
-    load_slot(t_lo + 1);
-    __syncthreads();
-    issue(t_lo);
-    hand_slot(t_lo + 1);
-    load_slot(t_lo + 2);
-    stage(t_lo & 1);
-    __syncthreads();
-    if (t_lo + 1 < t_hi) issue(t_lo + 1);
-    hand_slot(t_lo + 2);
-    load_slot(t_lo + 3);
-    __syncthreads();
-    for (int kb = t_lo; kb < t_hi; ++kb) {
-      tile(kb);
-      if (kb + 1 < t_hi) stage((kb + 1) & 1);
-      if (kb + 2 < t_hi) issue(kb + 2);
-      hand_slot(kb + 3);
-      load_slot(kb + 4);
+  } else {
+    int t0 = next(), t1 = next(), t2 = next(), t3 = next(), t4 = next();
+    if (t0 >= 0) {
+      load_slot(t0);
+      hand_slot(t0, 0);
+      load_slot(t1);
       __syncthreads();
+      issue(t0, 0);
+      hand_slot(t1, 1);
+      load_slot(t2);
+      stage(0);
+      __syncthreads();
+      if (t1 >= 0) issue(t1, 1);
+      hand_slot(t2, 0);
+      load_slot(t3);
+      __syncthreads();
+    }
+    for (int i = 0; t0 >= 0; ++i) {
+      tile(t0, i & 1);
+      if (t1 >= 0) stage(i + 1 & 1);
+      if (t2 >= 0) issue(t2, i & 1);
+      hand_slot(t3, i + 1 & 1);
+      load_slot(t4);
+      __syncthreads();
+      t0 = t1;
+      t1 = t2;
+      t2 = t3;
+      t3 = t4;
+      t4 = next();
     }
   }
   if (bad) flag_error(a.err, IR_ERR_GATHER_RANGE);
@@ -605,18 +835,20 @@ __global__ __launch_bounds__(256) void paged_masked_merge_kernel(MaskedArgs a) {
   const int64_t row = it / (D / 4);
   if (row >= per_part) return;
   const int d0 = (int)(it - row * (D / 4)) * 4;
+  const int rows = a.seq_q * a.n_rep;
+  const int64_t unit = row / rows;
+  const int r = (int)(row - unit * rows);
+  const int n_rtw = (rows + kWideCols - 1) / kWideCols;
+  const int parts = a.vis ? abs(a.walks[unit * n_rtw + r / kWideCols].x) : a.parts;
   PartMerge run;
 #pragma unroll 4
-  for (int p = 0; p < a.parts; ++p) {
+  for (int p = 0; p < parts; ++p) {
     const int64_t pr = p * per_part + row;
     const f32x2 ml = *(const f32x2*)(a.ws_ml + pr * 2);
     const f32x4 v = *(const f32x4*)(a.ws_o + pr * D + d0);
     const float x[4] = {v[0], v[1], v[2], v[3]};
     run.add(ml[0], ml[1], x);
   }
-  const int rows = a.seq_q * a.n_rep;
-  const int64_t unit = row / rows;
-  const int r = (int)(row - unit * rows);
   const int kvh = (int)(unit % a.num_kv_heads), b = (int)(unit / a.num_kv_heads);
   const int sq = r / a.n_rep;
   const int oh = kvh * a.n_rep + (r - sq * a.n_rep);
@@ -626,10 +858,12 @@ __global__ __launch_bounds__(256) void paged_masked_merge_kernel(MaskedArgs a) {
 
 // ---------------------------------------------------------------- host side
 
+constexpr int kSurveyParts = 12;
 constexpr int64_t kMaxPartBytes = 256ll << 20;  // bound of a call's partial rows
 
 struct Split {
   bool wide;
+  bool survey;  // the wide kernel may be told which tiles to leave out
   int64_t nwg;  // workgroups of one part
   int parts;    // parts that pay
 };
@@ -643,11 +877,29 @@ Split split_of(int64_t batch, int64_t seq_q, int64_t seq_k, int num_q_heads, int
   Split s;
   s.wide = rows > 32 && dtype != IR_DTYPE_F32 && (mask_dtype == dtype || mask_dtype == IR_DTYPE_F32) &&
            mask_t_stride == 1 && seq_k <= (1 << 28) && num_slots <= 0x7fffffff;
+  // (the survey pays for itself from about 1000 keys; its bytes stay small)
+  const int n_rep = num_q_heads / num_kv_heads;
+  s.survey = s.wide && mask_dtype == dtype && n_rep >= 5 && seq_k >= kSurveyMin * kTileKeys && seq_k <= (1 << 20);
   s.nwg = batch * num_kv_heads * (s.wide ? (rows + kWideCols - 1) / kWideCols : (rows + 15) / 16);
   const int64_t slots = (int64_t)device_cus() * 2;
   const int64_t units = s.wide ? (seq_k + kTileKeys - 1) / kTileKeys / 2 : (seq_k + 15) / 16 / (2 * kWaves);
   s.parts = (int)std::max<int64_t>(1, std::min<int64_t>({s.nwg > 0 ? slots / s.nwg : 1, units, 64}));
+  // surveyed walks differ in length; parts beyond a block's own need cost nothing
+  if (s.survey && s.nwg < 2 * slots) s.parts = std::max(s.parts, (int)std::min<int64_t>(units, kSurveyParts));
   return s;
+}
+
+// Bytes of a surveyed call's vis, tok_vis, walks and bounds (each 256-byte aligned).
+struct SurveyBytes {
+  int64_t vis, tok_vis, walks, bounds;
+  int64_t total() const { return vis + tok_vis + walks + bounds; }
+};
+SurveyBytes survey_bytes(const Split& sp, int64_t batch, int64_t seq_k, int num_kv_heads) {
+  if (!sp.survey) return {0, 0, 0, 0};
+  const int64_t nt = (seq_k + kTileKeys - 1) / kTileKeys, blocks = sp.nwg / num_kv_heads;  // of all sequences
+  auto up = [](int64_t x) { return (x + 255) / 256 * 256; };
+  return {up(blocks * ((nt + 63) / 64 * 64)), up(blocks * ((nt + kSurveyTiles - 1) / kSurveyTiles) * 32),
+          up(sp.nwg * 8), up(batch * num_kv_heads * nt * 4)};
 }
 
 int64_t part_bytes(int64_t batch, int64_t seq_q, int num_q_heads, int head_dim) {
@@ -661,9 +913,15 @@ void launch(const MaskedArgs& a, const Split& sp, hipStream_t s) {
     if (sp.wide) {
       if (a.mask_dtype == IR_DTYPE_F32)
         hipLaunchKernelGGL((paged_masked_wide_kernel<DT, D, 4, false>), grid, block, 0, s, a);
-      else if (a.n_rep >= 5)
+      else if (a.n_rep >= 5) {
+        if (a.vis) {
+          const int nt = (a.seq_k + kTileKeys - 1) / kTileKeys, n_rtw = (int)(sp.nwg / a.num_kv_heads / a.batch);
+          const int64_t wgs = (int64_t)a.batch * (a.num_kv_heads * nt + n_rtw * ((nt + kSurveyTiles - 1) / kSurveyTiles));
+          hipLaunchKernelGGL((paged_masked_survey_kernel<DT, D>), dim3((unsigned)wgs), dim3(256), 0, s, a, nt, n_rtw);
+          hipLaunchKernelGGL((paged_masked_walks_kernel<DT, D>), dim3((unsigned)sp.nwg), dim3(256), 0, s, a, nt, n_rtw);
+        }
         hipLaunchKernelGGL((paged_masked_wide_kernel<DT, D, 2, true>), grid, block, 0, s, a);
-      else
+      } else
         hipLaunchKernelGGL((paged_masked_wide_kernel<DT, D, 2, false>), grid, block, 0, s, a);
     }
   }
@@ -693,7 +951,7 @@ extern "C" int64_t ir_paged_attention_masked_workspace_size(int batch, int seq_q
   const Split sp = split_of(batch, seq_q, seq_k, num_q_heads, num_kv_heads, dtype, mask_dtype, mask_t_stride, 0);
   const int64_t per = part_bytes(batch, seq_q, num_q_heads, head_dim);
   const int64_t parts = std::min<int64_t>(sp.parts, kMaxPartBytes / per);
-  return parts > 1 ? parts * per : 0;
+  return (parts > 1 ? parts * per : 0) + survey_bytes(sp, batch, seq_k, num_kv_heads).total();
 }
 
 extern "C" int ir_paged_attention_masked(const void* q, int64_t q_b_stride, int64_t q_s_stride,
@@ -787,9 +1045,23 @@ extern "C" int ir_paged_attention_masked_ws(const void* q, int64_t q_b_stride, i
   // per layer): it stays one launch, each workgroup taking the parts of the
   // ungated call one after the other, with the same bits.
   a.serial = run_if && !sp.wide;
-  const int64_t room = a.serial ? kMaxPartBytes : workspace ? workspace_bytes : 0;
+  // The survey's bytes come first; a workspace too small for them goes without.
+  const SurveyBytes sv = survey_bytes(sp, batch, seq_k, num_kv_heads);
+  const bool survey = sv.total() > 0 && workspace && workspace_bytes >= sv.total() && num_slots > 0;
+  uint8_t* ws = (uint8_t*)workspace;
+  a.vis = a.tok_vis = nullptr;
+  a.walks = nullptr;
+  a.bounds = nullptr;
+  if (survey) {
+    a.vis = ws;
+    a.tok_vis = a.vis + sv.vis;
+    a.walks = (int2*)(a.tok_vis + sv.tok_vis);
+    a.bounds = (float*)((uint8_t*)a.walks + sv.walks);
+    ws += sv.total();
+  }
+  const int64_t room = a.serial ? kMaxPartBytes : workspace ? workspace_bytes - (survey ? sv.total() : 0) : 0;
   a.parts = (int)std::max<int64_t>(1, std::min<int64_t>(sp.parts, room / per));
-  a.ws_o = (float*)workspace;
+  a.ws_o = (float*)ws;
   a.ws_ml = a.ws_o + (int64_t)a.parts * batch * seq_q * num_q_heads * head_dim;
   IR_REQUIRE(sp.nwg * a.parts < (1ll << 31), "ir_paged_attention_masked: grid too large");
   hipStream_t s = (hipStream_t)stream;

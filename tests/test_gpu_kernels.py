@@ -509,6 +509,74 @@ def test_masked_kernels_at_their_edges(b, sq, t, h_kv, n_rep, d, dtype, mask_dty
     assert bool((gated == 7.0).all())
 
 
+@pytest.mark.parametrize("change", ["none", "row masked", "large scores", "nan in v", "inf in k", "bad slot", "faint bias"])
+@pytest.mark.parametrize("n_rep,d,dtype,lens", [
+    (7, 128, torch.bfloat16, [(900, 1), (30, 40), (0, 129), (64, 64)]),
+    (7, 64, torch.float16, [(0, 64), (4100, 3), (64, 20)]),
+])
+def test_masked_survey_leaves_out_only_what_adds_nothing(n_rep, d, dtype, lens, change):
+    """A long packed frame with the block-diagonal varlen mask, and every reason not to
+    leave a tile out: a row without a visible key, scores that reach past the mask,
+    values that are not finite, a slot outside the pool, a row that sees only a large
+    negative bias. Held against the same call without a workspace (no survey, every
+    tile walked) and, where the values are finite, the oracle."""
+    from infrared_amd._lib import check, dtype_code, lib, ptr, stream_ptr
+
+    h_kv, slots_n = 2, 6000
+    q_seq, q_pos, k_seq, k_pos = [], [], [], []
+    for i, (start, n) in enumerate(lens):
+        q_seq += [i] * n
+        q_pos += range(start, start + n)
+        k_seq += [i] * (start + n)
+        k_pos += range(start + n)
+    g = torch.Generator().manual_seed(d)
+    sq, t = len(q_seq), len(k_seq)
+    assert t >= 1024
+    mask = O.varlen_mask(torch.tensor(q_seq), torch.tensor(q_pos), torch.tensor(k_seq), torch.tensor(k_pos), dtype)
+    gs = torch.randperm(slots_n, generator=g)[:t][None]
+    kc = torch.randn(slots_n, h_kv, d, generator=g).to(dtype)
+    vc = torch.randn(slots_n, h_kv, d, generator=g).to(dtype)
+    q = torch.randn(1, sq, h_kv * n_rep, d, generator=g).to(dtype)
+    if change == "row masked":
+        mask[0, 0, sq // 2] = torch.finfo(dtype).min
+    elif change == "large scores":
+        q *= 3000.0
+        kc *= 40.0
+    elif change == "nan in v":
+        vc[gs[0, 5]] = float("nan")
+    elif change == "inf in k":
+        kc[gs[0, 5], :, 3] = float("inf")
+    elif change == "faint bias":
+        mask[0, 0, sq // 2] = torch.finfo(dtype).min
+        mask[0, 0, sq // 2, t // 2] = -5e4
+    ref = None
+    if change in ("none", "row masked", "faint bias"):
+        ref = O.paged_attention_naive(q.float(), kc.float(), vc.float(), gs, mask.float(), d**-0.5, n_rep)
+    if change == "bad slot":
+        gs[0, 7] = slots_n
+    q, kc, vc, gs, mask = (x.to(DEV) for x in (q, kc, vc, gs, mask))
+    err = _err()
+    out = kernels.paged_attention_masked(q, kc, vc, gs, mask, d**-0.5, err_flags=err)
+    assert err.item() == (ERR_GATHER_RANGE if change == "bad slot" else 0)
+    dense = torch.empty_like(out)
+    check(lib().ir_paged_attention_masked_ws(
+        ptr(q), q.stride(0), q.stride(1), q.stride(2), ptr(kc), ptr(vc), kc.stride(0), kc.stride(1), kc.shape[0],
+        ptr(gs), gs.stride(0), gs.stride(1), ptr(mask), mask.stride(0), mask.stride(2), mask.stride(3),
+        dtype_code(dtype), ptr(dense), *dense.stride()[:3], 1, sq, t, h_kv * n_rep, h_kv, d, d**-0.5,
+        dtype_code(dtype), None, None, None, 0, stream_ptr(out.device)), "ir_paged_attention_masked_ws")
+    assert torch.equal(out.isnan(), dense.isnan())
+    # Each call rounds every probability to dtype (half an eps) relative to its own parts'
+    # running maxima, so the two differ by at most eps * sum(p |v|) / sum(p) <= eps * max |v|,
+    # and by the rounding of the output, eps * |out|.
+    eps = torch.finfo(dtype).eps
+    vmax = vc[vc.isfinite()].abs().max().item()
+    assert torch.allclose(out.float(), dense.float(), rtol=eps, atol=eps * vmax, equal_nan=True)
+    if change == "nan in v":
+        assert bool(out.isnan().any())
+    if ref is not None:
+        assert (out.float().cpu() - ref).abs().max().item() <= TOL[dtype]
+
+
 def test_config_table_is_consistent():
     for name, cfg in DECODE_CONFIGS.items():
         assert cfg.num_q_heads % cfg.num_kv_heads == 0, name
