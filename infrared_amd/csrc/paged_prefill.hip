@@ -1542,15 +1542,19 @@ PrefillGeometry prefill_geometry(int max_q_len, int n_rep) {
   return g;
 }
 
-// The fp32 kernel's items: 64 columns, two workgroups resident per CU
-// (n_rep <= kF32Cols).
-PrefillGeometry prefill_geometry_f32(int max_q_len, int n_rep) {
+// The fp32 kernel's items: 64 columns (n_rep <= kF32Cols). Two workgroups are
+// resident per CU at head_dim 128 and three at 64 (73 and 39 KB of LDS, 130
+// registers), and 64-column workgroups are short of wavefronts to hide their
+// loads: at 64 the plan cuts for four (6 chunks of 64..512 tokens after up to
+// 1500, 14/2 heads: 61.8 us a layer against 66.1 cut for two; four resident at 128
+// registers: the same 61.8).
+PrefillGeometry prefill_geometry_f32(int max_q_len, int n_rep, int head_dim) {
   PrefillGeometry g;
   g.nw = 4;
   g.tq = kF32Cols / n_rep;
   g.n_qblocks = (max_q_len + g.tq - 1) / g.tq;
   g.sched = kRing2;
-  g.slots = 2 * device_cus();
+  g.slots = (head_dim == 64 ? 4 : 2) * device_cus();
   g.cols = kF32Cols;
   return g;
 }
@@ -1656,7 +1660,7 @@ extern "C" int64_t ir_paged_prefill_plan_bytes(int num_seqs, int max_q_len, int 
   const int n_rep = num_q_heads / num_kv_heads;
   const int64_t b16 = plan_layout(prefill_geometry(max_q_len, n_rep), num_seqs, num_kv_heads, head_dim).total;
   if (n_rep > kF32Cols) return b16;
-  return std::max(b16, plan_layout(prefill_geometry_f32(max_q_len, n_rep), num_seqs, num_kv_heads, head_dim).total);
+  return std::max(b16, plan_layout(prefill_geometry_f32(max_q_len, n_rep, head_dim), num_seqs, num_kv_heads, head_dim).total);
 }
 
 extern "C" int ir_paged_prefill_plan_xcds(void) { return plan_xcds(); }
@@ -1719,7 +1723,7 @@ extern "C" int ir_paged_prefill(const void* q, int64_t q_tok_stride, int64_t q_h
   a.num_seqs = num_seqs;
   a.total_q = total_q;
   a.n_rep = num_q_heads / num_kv_heads;
-  const PrefillGeometry geo = f32 ? prefill_geometry_f32(max_q_len, a.n_rep) : prefill_geometry(max_q_len, a.n_rep);
+  const PrefillGeometry geo = f32 ? prefill_geometry_f32(max_q_len, a.n_rep, head_dim) : prefill_geometry(max_q_len, a.n_rep);
   a.nw = geo.nw;
   a.tq = geo.tq;
   a.n_qblocks = geo.n_qblocks;
@@ -1801,7 +1805,7 @@ extern "C" int ir_paged_prefill_plan(const int32_t* cu_seqlens_q, const int32_t*
   IR_REQUIRE(bt_stride >= max_blocks_per_seq, "ir_paged_prefill_plan: bt_stride %lld below max_blocks_per_seq %d",
              (long long)bt_stride, max_blocks_per_seq);
   const int n_rep = num_q_heads / num_kv_heads;
-  const PrefillGeometry geo = f32 ? prefill_geometry_f32(max_q_len, n_rep) : prefill_geometry(max_q_len, n_rep);
+  const PrefillGeometry geo = f32 ? prefill_geometry_f32(max_q_len, n_rep, head_dim) : prefill_geometry(max_q_len, n_rep);
   const PlanLayout ly = plan_layout(geo, num_seqs, num_kv_heads, head_dim);
   IR_REQUIRE(ly.entries <= 0x7fffffff && ly.cap_pieces < 65536 &&
                  (int64_t)num_seqs * geo.n_qblocks * num_kv_heads <= 0x7fffffff &&
