@@ -4,12 +4,12 @@ Same API as the reference module:
 
 - ``default_buckets`` / ``pick_bucket`` (``infrared/engine/cuda_graph.py:58-81``);
 - ``build_decode_static_inputs`` (``:105-155``): fixed-shape inputs for a batch
-  bucket, pad-by-repeating row 0, key axis padded to ``t_max``. Built
-  by one kernel (``ir_decode_inputs``) instead of a Python loop over ``B * ctx`` tokens, and
-  carrying the ``block_tables``/``context_lens`` the HIP decode kernel reads;
+  bucket, pad-by-repeating row 0, key axis padded to ``t_max``. Built by one
+  kernel (``ir_decode_inputs``) instead of a Python loop over ``B * ctx``
+  tokens, and carrying the ``block_tables``/``context_lens`` the HIP decode kernel reads;
 - ``HipGraphDecoder`` (in place of ``CudaGraphDecoder``, ``:170-287``): one
-  captured graph per bucket sharing one memory pool; ``decode()`` copies the
-  step's metadata into the static buffers and replays.
+  captured graph per bucket sharing one memory pool; ``decode()`` builds the
+  step's metadata in the static buffers and replays.
 
 PyTorch-ROCm's ``torch.cuda.CUDAGraph`` is a hipGraph; the HIP kernels are
 launched on torch's current stream, so they are captured as graph kernel

@@ -466,6 +466,7 @@ def test_masked_fully_masked_row_is_uniform_and_bad_slot_flagged():
     (1, 130, 200, 1, 1, 64, torch.float16, torch.float16),    # one head a token
     (1, 27, 130, 1, 5, 128, torch.bfloat16, torch.bfloat16),  # 5 heads: 27 tokens in a workgroup
     (1, 9, 4200, 1, 40, 64, torch.bfloat16, torch.bfloat16),  # 40 heads a token
+    (2, 40, 1100, 2, 7, 128, torch.float16, torch.float16),   # two sequences, surveyed
 ])
 @pytest.mark.parametrize("strided", [False, True])
 def test_masked_kernels_at_their_edges(b, sq, t, h_kv, n_rep, d, dtype, mask_dtype, strided):
