@@ -335,6 +335,17 @@ def test_decode_flags_bad_block_ids_and_contexts():
     assert err.item() & ERR_CONTEXT_RANGE
 
 
+def test_native_calls_refuse_a_zero_block_size():
+    """A division in the native binding must not take the process down."""
+    case = make_decode_case("qwen7b-bf16", DEV, num_seqs=2)
+    bt, cl = case.block_tables[0], case.context_lens
+    with pytest.raises(RuntimeError, match="block_size"):
+        kernels.paged_decode(case.q, case.k_cache, case.v_cache, bt, cl, 0, 0.1)
+    cu = torch.tensor([0, 1, 2], dtype=torch.int32, device=DEV)
+    with pytest.raises(RuntimeError, match="block_size"):
+        kernels.paged_prefill(case.q, case.k_cache, case.v_cache, bt, cu, cl, 1, 0, 0.1)
+
+
 def test_decode_one_hot_probe_returns_exact_v_row():
     """A key whose score dwarfs the rest makes the output equal its V row, which pins
     the block-table address of that key exactly."""
