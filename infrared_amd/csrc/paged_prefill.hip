@@ -1212,7 +1212,7 @@ struct PlanArgs {
   const int32_t* bt;  // block tables: the first id of each row groups shared prefixes
   int64_t bt_stride;
   int num_seqs, total_q, n_qblocks, tq, cap, bs;  // cap: keys the block tables hold
-  int num_kv_heads, slots, cap_pieces, xcds;      // slots: workgroups resident on the device at once
+  int num_kv_heads, slots, cap_pieces, xcds;      // slots: workgroups whose mean load is the cut threshold
   int share_groups;   // place share groups on slots of XCDs (else one global order)
   int entries;        // workgroups of a planned call
   int2* items;        // [entries]
@@ -1525,6 +1525,7 @@ int plan_xcds() {
 // columns or on request. `slots`: workgroups resident at once.
 struct PrefillGeometry {
   int nw, tq, n_qblocks, sched, slots, cols;  // cols: query columns (token x head) of a work item
+  int cut_slots;  // workgroups the plan's cut threshold is the mean load of (slots bounds its pieces)
 };
 
 PrefillGeometry prefill_geometry(int max_q_len, int n_rep) {
@@ -1538,7 +1539,7 @@ PrefillGeometry prefill_geometry(int max_q_len, int n_rep) {
   // lockstep form needs more than 256 and spilled)
   const bool ring2 = g.nw == 8 || k.ring2 != 0;
   g.sched = ring2 ? kRing2 : kLockstep;
-  g.slots = ring2 && g.nw == 4 ? 2 * cus : cus;
+  g.slots = g.cut_slots = ring2 && g.nw == 4 ? 2 * cus : cus;
   g.cols = 32 * g.nw;
   return g;
 }
@@ -1546,16 +1547,18 @@ PrefillGeometry prefill_geometry(int max_q_len, int n_rep) {
 // The fp32 kernel's items: 64 columns (n_rep <= kF32Cols). Two workgroups are
 // resident per CU at head_dim 128 and three at 64 (73 and 39 KB of LDS, 130
 // registers), and 64-column workgroups are short of wavefronts to hide their
-// loads: at 64 the plan cuts for four (6 chunks of 64..512 tokens after up to
-// 1500, 14/2 heads: 61.8 us a layer against 66.1 cut for two; four resident at 128
-// registers: the same 61.8).
+// loads, so at 64 the plan cuts for three (6 chunks of 64..512 tokens after up to
+// 1500, 14/2 heads, per layer: 63.8 us against 66.1 cut for two; cut for four
+// 64.6, as the pieces then exceed the plan's capacity and the threshold rises
+// again). The capacity stays that of two per CU.
 PrefillGeometry prefill_geometry_f32(int max_q_len, int n_rep, int head_dim) {
   PrefillGeometry g;
   g.nw = 4;
   g.tq = kF32Cols / n_rep;
   g.n_qblocks = (max_q_len + g.tq - 1) / g.tq;
   g.sched = kRing2;
-  g.slots = (head_dim == 64 ? 4 : 2) * device_cus();
+  g.slots = 2 * device_cus();
+  g.cut_slots = (head_dim == 64 ? 3 : 2) * device_cus();
   g.cols = kF32Cols;
   return g;
 }
@@ -1824,7 +1827,7 @@ extern "C" int ir_paged_prefill_plan(const int32_t* cu_seqlens_q, const int32_t*
   p.cap = max_blocks_per_seq * block_size;
   p.bs = block_size;
   p.num_kv_heads = num_kv_heads;
-  p.slots = geo.slots;
+  p.slots = geo.cut_slots;
   p.cap_pieces = prefill_knobs().cuts ? (int)ly.cap_pieces : 0;
   p.xcds = plan_xcds();
   p.share_groups = (flags & IR_PLAN_SHARE_GROUPS) != 0;
