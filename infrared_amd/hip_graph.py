@@ -156,6 +156,9 @@ def _fill_inputs(out: DecodeInputs, block_tables: Sequence[Sequence[int]], num_c
         ptr(out.positions), ptr(out.write_slots), ptr(out.gather_slots), ptr(out.mask), ptr(out.block_tables),
         ptr(out.context_lens), stream_ptr(dev),
     ), "ir_decode_inputs")
+    # written through raw pointers: what is cached of these tensors (the pool's
+    # reference-form check of gather_slots and mask) has to see that they changed
+    torch.autograd.graph.increment_version([getattr(out, n) for n in DecodeInputs.__slots__])
 
 
 @dataclass(slots=True)

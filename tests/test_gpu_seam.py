@@ -898,3 +898,33 @@ def test_prefill_context_slots_match_the_per_token_slots(num_cached, q_lens):
         assert s.dec_ctx.tolist() == [num_cached[i] + 1 for i in dec]
         assert s.pre_q_start.tolist() == [num_cached[i] for i in pre]
         assert s.pre_cu.tolist() == [sum(q_lens[i] for i in pre[:j]) for j in range(len(pre) + 1)]
+
+
+def test_reference_form_check_sees_refilled_graph_buffers():
+    """A step function that attends in the reference form, then the same call made
+    eagerly on the captured buffers after each decode() has refilled them: the form
+    cached from the warm-up (or the last call) is not taken for the new step's."""
+    bs, h_kv, n_rep, d, t_max = 16, 4, 7, 128, 256
+    dtype = torch.bfloat16
+    pool = PagedKVPool(1, 64, bs, h_kv, d, dtype, device=DEV)
+    pool.k.normal_()
+    pool.v.normal_()
+    gen = torch.Generator(device=DEV).manual_seed(9)
+    q, k, v = (torch.randn(2, 1, h, d, generator=gen, device=DEV).to(dtype) for h in (h_kv * n_rep, h_kv, h_kv))
+    bufs = {}
+
+    def step(buf, paged):
+        bufs["now"] = buf
+        return paged_attention(q, k, v, _ReferenceContext(pool, buf.write_slots, buf.gather_slots), buf.mask, 0,
+                               d**-0.5, n_rep)
+
+    dec = HipGraphDecoder(None, pool, max_num_seqs=2, t_max=t_max, block_size=bs, step_fn=step)
+    tables = [list(range(16)), list(range(32, 48))]
+    for num_cached in ([20, 200], [150, 30], [21, 201]):
+        replayed = dec.decode(tables, num_cached, [0, 0]).clone()
+        eager = step(bufs["now"], None)
+        want = O.paged_attention_naive(
+            q.float().cpu(), pool.k[0].float().cpu(), pool.v[0].float().cpu(), bufs["now"].gather_slots.cpu(),
+            bufs["now"].mask.float().cpu(), d**-0.5, n_rep)
+        for got in (replayed, eager):
+            assert (got.float().cpu() - want).abs().max().item() <= 2e-2, num_cached

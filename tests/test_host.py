@@ -210,3 +210,21 @@ def test_record_wait_returns_once_the_tag_is_there():
     host = np.zeros(16, dtype=np.int32)
     host[7] = 12345
     kernels.await_record(host, 7, 12345, torch.device("cuda"))
+
+
+def test_refilled_static_inputs_count_as_modified(monkeypatch):
+    """The native fill writes the static buffers through raw pointers; their version
+    counters move as a copy_ would move them, since the pool's form checks are cached
+    on them."""
+    class Recorder:
+        def ir_decode_inputs(self, *args):
+            return 0
+
+    monkeypatch.setattr(hip_graph, "lib", Recorder)
+    monkeypatch.setattr(hip_graph, "to_device", lambda host, device: torch.from_numpy(host))
+    monkeypatch.setattr(hip_graph, "stream_ptr", lambda device: 0)
+    buf = hip_graph.build_decode_static_inputs([[1], [2]], [3, 4], [7, 8], 2, 32, 16, "cpu", torch.float32)
+    before = {n: getattr(buf, n)._version for n in type(buf).__slots__}
+    hip_graph._fill_inputs(buf, [[1], [2]], [4, 5], [9, 9], 16)
+    for n, v in before.items():
+        assert getattr(buf, n)._version > v, n
