@@ -91,7 +91,8 @@ def build_decode_static_inputs(
     ``slot(bt_i, num_cached[i])``) and attends ``[0, num_cached[i]]``.
     """
     device = torch.device(device)
-    b = _check_rows(num_cached, last_tokens, bucket_b, t_max)
+    num_cached, last_tokens = _check_rows(num_cached, last_tokens, bucket_b, t_max)
+    b = len(last_tokens)
     width = metadata.blocks_for(t_max, block_size)
     if device.type == "cuda" and dtype in _MASK_DTYPES and bucket_b < 65536:
         out = DecodeInputs(
@@ -126,27 +127,31 @@ def build_decode_static_inputs(
 _MASK_DTYPES = (torch.float32, torch.float16, torch.bfloat16)
 
 
-def _check_rows(num_cached: Sequence[int], last_tokens: Sequence[int], bucket_b: int, t_max: int) -> int:
-    """The rows of a step that fits ``(bucket_b, t_max)``; raises otherwise."""
+def _check_rows(num_cached: Sequence[int], last_tokens: Sequence[int], bucket_b: int,
+                t_max: int) -> tuple[list[int], list[int]]:
+    """The cached lengths and last tokens of a step that fits ``(bucket_b,
+    t_max)``, one of each per row; raises otherwise."""
     b = len(last_tokens)
     if not 0 < b <= bucket_b:
         raise ValueError(f"need 0 < b ({b}) <= bucket_b ({bucket_b})")
-    for n in num_cached[:b]:
+    cached = [num_cached[j] for j in range(b)]  # (IndexError if one is missing)
+    for n in cached:
         if n < 0:
             raise ValueError(f"num_cached {n} is negative")
         if n + 1 > t_max:
             raise ValueError(f"context_len {n + 1} exceeds t_max {t_max}")
-    return b
+    return cached, list(last_tokens)
 
 
-def _fill_inputs(out: DecodeInputs, block_tables: Sequence[Sequence[int]], num_cached: Sequence[int],
-                 last_tokens: Sequence[int], block_size: int) -> None:
-    """Writes a step's inputs into ``out`` (device tensors, contiguous): one
-    host array, one copy, one launch (``ir_decode_inputs``)."""
+def _fill_inputs(out: DecodeInputs, block_tables: Sequence[Sequence[int]], num_cached: list[int],
+                 last_tokens: list[int], block_size: int) -> None:
+    """Writes a step's inputs (lengths and tokens as ``_check_rows`` gives them)
+    into ``out`` (device tensors, contiguous): one host array, one copy, one
+    launch (``ir_decode_inputs``)."""
     b, (bucket_b, width) = len(last_tokens), out.block_tables.shape
     host = np.zeros(4 * b + b * width, dtype=np.int32)
     rows = host[: 4 * b].view(np.int64).reshape(b, 2)
-    rows[:, 0] = num_cached[:b]
+    rows[:, 0] = num_cached
     rows[:, 1] = last_tokens
     metadata.fill_tables(host[4 * b :].reshape(b, width), [list(block_tables[j])[:width] for j in range(b)])
     dev = out.mask.device
@@ -215,8 +220,8 @@ class HipGraphDecoder:
         b = len(last_tokens)
         bucket = pick_bucket(b, self.buckets)
         if bucket in self._graphs and self.dtype in _MASK_DTYPES and bucket < 65536:
-            _check_rows(num_cached, last_tokens, bucket, self.t_max)
-            _fill_inputs(self._graphs[bucket].buf, block_tables, num_cached, last_tokens, self.block_size)
+            cached, tokens = _check_rows(num_cached, last_tokens, bucket, self.t_max)
+            _fill_inputs(self._graphs[bucket].buf, block_tables, cached, tokens, self.block_size)
         else:
             inp = build_decode_static_inputs(
                 block_tables, num_cached, last_tokens, bucket, self.t_max, self.block_size,

@@ -228,3 +228,22 @@ def test_refilled_static_inputs_count_as_modified(monkeypatch):
     hip_graph._fill_inputs(buf, [[1], [2]], [4, 5], [9, 9], 16)
     for n, v in before.items():
         assert getattr(buf, n)._version > v, n
+
+
+def test_a_missing_cached_length_is_refused():
+    """Fewer cached lengths than rows, one among them (numpy would repeat it for every
+    row): an IndexError before anything is written, from the build and the refill alike."""
+    with pytest.raises(IndexError):
+        hip_graph.build_decode_static_inputs([[1], [2], [3]], [5], [7, 8, 9], 4, 32, 16, "cpu", torch.float32)
+
+    class Captured:
+        buf = None
+
+    pool = type("Pool", (), {"device": torch.device("cpu"), "dtype": torch.float32})()
+    dec = hip_graph.HipGraphDecoder(None, pool, max_num_seqs=4, t_max=32, block_size=16)
+    dec._graphs[4] = Captured()
+    with pytest.raises(IndexError):
+        dec.decode([[1], [2], [3]], [5], [7, 8, 9])
+    # more lengths than rows: the first ones count, as before
+    inp = hip_graph.build_decode_static_inputs([[1], [2]], [5, 6, 7], [7, 8], 2, 32, 16, "cpu", torch.float32)
+    assert inp.context_lens.tolist() == [6, 7]
