@@ -32,7 +32,7 @@ import torch
 
 from infrared_amd import metadata
 from infrared_amd._lib import check, dtype_code, lib, ptr, stream_ptr
-from infrared_amd.paged_kv_cache import PagedContext, PagedKVPool, to_device
+from infrared_amd.paged_kv_cache import PagedContext, PagedKVPool, host_list, to_device
 
 
 def default_buckets(max_num_seqs: int) -> tuple[int, ...]:
@@ -134,13 +134,14 @@ def _check_rows(num_cached: Sequence[int], last_tokens: Sequence[int], bucket_b:
     b = len(last_tokens)
     if not 0 < b <= bucket_b:
         raise ValueError(f"need 0 < b ({b}) <= bucket_b ({bucket_b})")
-    cached = [num_cached[j] for j in range(b)]  # (IndexError if one is missing)
+    cached = host_list(num_cached)
+    cached = [int(cached[j]) for j in range(b)]  # (IndexError if one is missing)
     for n in cached:
         if n < 0:
             raise ValueError(f"num_cached {n} is negative")
         if n + 1 > t_max:
             raise ValueError(f"context_len {n + 1} exceeds t_max {t_max}")
-    return cached, list(last_tokens)
+    return cached, [int(t) for t in host_list(last_tokens)]
 
 
 def _fill_inputs(out: DecodeInputs, block_tables: Sequence[Sequence[int]], num_cached: list[int],

@@ -20,12 +20,13 @@ decode kernel reads, so a caller fills ``PagedContext`` directly:
 from __future__ import annotations
 
 from collections.abc import Sequence
+from operator import index
 
 import numpy as np
 import torch
 
 from infrared_amd._lib import check, lib, ptr, stream_ptr
-from infrared_amd.paged_kv_cache import PagedContext, PagedKVPool, row_split, to_device
+from infrared_amd.paged_kv_cache import PagedContext, PagedKVPool, host_list, row_split, to_device
 
 
 def slot(block_table: Sequence[int], pos: int, block_size: int) -> int:
@@ -165,6 +166,7 @@ def prefill_context(
     bs = pool.block_size
     if not (len(block_tables) == len(num_cached) == len(q_lens)):
         raise ValueError("block_tables, num_cached and q_lens must have one entry per sequence")
+    num_cached, q_lens = [[index(n) for n in host_list(x)] for x in (num_cached, q_lens)]
     lengths = [c + n for c, n in zip(num_cached, q_lens)]
     width = max(blocks_for(n, bs) for n in lengths) if lengths else 0
     rows = [r[: max(width, 1)] for r in block_tables]

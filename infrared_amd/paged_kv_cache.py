@@ -436,6 +436,12 @@ def row_split(bt: torch.Tensor, num_cached: Sequence[int], q_lens: Sequence[int]
     )
 
 
+def host_list(values: Sequence[int] | torch.Tensor) -> list:
+    """The step's numbers as a list on the host: a sequence, or a tensor wherever
+    it lives (sampled tokens, say), read in one copy."""
+    return values.reshape(-1).tolist() if torch.is_tensor(values) else list(values)
+
+
 def to_device(host: np.ndarray, device: torch.device) -> torch.Tensor:
     """A host array on ``device`` through pinned staging memory (torch's caching
     allocator keeps it until the copy has run), so the host does not wait for

@@ -928,3 +928,29 @@ def test_reference_form_check_sees_refilled_graph_buffers():
             bufs["now"].mask.float().cpu(), d**-0.5, n_rep)
         for got in (replayed, eager):
             assert (got.float().cpu() - want).abs().max().item() <= 2e-2, num_cached
+
+
+def test_step_metadata_takes_numbers_from_the_device():
+    """Cached lengths, chunk lengths and last tokens as tensors on the device (sampled
+    tokens as argmax leaves them), as lists of such scalars, or as numpy arrays."""
+    c, t = [3, 20], [7, 8]
+    dc, dt = torch.tensor(c, device=DEV), torch.tensor(t, device=DEV)
+    tables = [[1], [2, 3]]
+    want = build_decode_static_inputs(tables, c, t, 4, 32, 16, "cpu", torch.float32)
+    for cached, tokens in ((dc, dt), (c, list(dt)), (list(dc), dt[:, None]), (dc.cpu().numpy(), dt.cpu())):
+        got = build_decode_static_inputs(tables, cached, tokens, 4, 32, 16, DEV, torch.float32)
+        for name in type(want).__slots__:
+            assert torch.equal(getattr(got, name).cpu(), getattr(want, name)), name
+    pool = PagedKVPool(1, 64, 16, 1, 64, torch.float32, device=DEV)
+    dec = HipGraphDecoder(None, pool, max_num_seqs=2, t_max=32, block_size=16, step_fn=lambda buf, paged: buf.ids + 1)
+    for _ in range(2):  # captured, then refilled
+        assert dec.decode(tables, dc, dt).tolist() == [[8], [9]]
+        dt = dt + 1
+        assert dec.decode(tables, list(dc), list(dt)).tolist() == [[9], [10]]
+        dt = dt - 1
+    ref, _ = metadata.prefill_context(pool, tables, c, [1, 3])
+    for cached, lens in ((dc, torch.tensor([1, 3], device=DEV)), (dc.cpu().numpy(), list(torch.tensor([1, 3])))):
+        got, _ = metadata.prefill_context(pool, tables, cached, lens)
+        assert got.max_q_len == 3 and got.row_split is not None
+        for name in ("write_slots", "block_tables", "cu_seqlens_q", "q_start"):
+            assert torch.equal(getattr(got, name), getattr(ref, name)), name
