@@ -445,10 +445,14 @@ def host_list(values: Sequence[int] | torch.Tensor) -> list:
 def to_device(host: np.ndarray, device: torch.device) -> torch.Tensor:
     """A host array on ``device`` through pinned staging memory (torch's caching
     allocator keeps it until the copy has run), so the host does not wait for
-    the stream as a copy from pageable memory does."""
+    the stream as a copy from pageable memory does. Under stream capture it
+    raises, as that copy did: a replay would read the staging memory again,
+    which belongs to someone else by then."""
     t = torch.from_numpy(host)
     if torch.device(device).type != "cuda":
         return t.to(device)
+    if torch.cuda.is_current_stream_capturing():
+        raise RuntimeError("a step's host metadata cannot be copied to the device while its stream is capturing")
     return torch.empty(t.shape, dtype=t.dtype, pin_memory=True).copy_(t).to(device, non_blocking=True)
 
 

@@ -954,3 +954,17 @@ def test_step_metadata_takes_numbers_from_the_device():
         assert got.max_q_len == 3 and got.row_split is not None
         for name in ("write_slots", "block_tables", "cu_seqlens_q", "q_start"):
             assert torch.equal(getattr(got, name), getattr(ref, name)), name
+
+
+def test_step_metadata_from_the_host_is_refused_under_capture():
+    pool = PagedKVPool(1, 64, 16, 1, 64, torch.float32, device=DEV)
+    x = torch.zeros(4, device=DEV)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        x += 1
+        with pytest.raises(RuntimeError, match="capturing"):
+            metadata.prefill_context(pool, [[1]], [3], [2])
+        with pytest.raises(RuntimeError, match="capturing"):
+            build_decode_static_inputs([[1]], [3], [7], 1, 32, 16, DEV, torch.float32)
+    graph.replay()
+    assert x.tolist() == [1.0] * 4  # the refusals left the capture whole

@@ -4,10 +4,11 @@ and the oracle's loop restatements."""
 
 from __future__ import annotations
 
+import numpy as np
 import pytest
 import torch
 
-from infrared_amd import hip_graph, metadata
+from infrared_amd import hip_graph, metadata, paged_kv_cache
 from oracle import naive as O
 
 
@@ -247,3 +248,12 @@ def test_a_missing_cached_length_is_refused():
     # more lengths than rows: the first ones count, as before
     inp = hip_graph.build_decode_static_inputs([[1], [2]], [5, 6, 7], [7, 8], 2, 32, 16, "cpu", torch.float32)
     assert inp.context_lens.tolist() == [6, 7]
+
+
+def test_host_metadata_is_refused_under_capture(monkeypatch):
+    """A copy from pinned staging memory would be recorded and replayed from memory
+    that has been handed out again: refused before anything is allocated."""
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    with pytest.raises(RuntimeError, match="capturing"):
+        paged_kv_cache.to_device(np.zeros(4, dtype=np.int32), "cuda")
+    assert paged_kv_cache.to_device(np.arange(3), "cpu").tolist() == [0, 1, 2]
