@@ -271,6 +271,8 @@ Tensor paged_prefill(const Tensor& q, const Tensor& kc, const Tensor& vc, const 
   const Tensor out = out_ ? *out_ : at::empty(q.sizes(), q.options());
   int64_t n_write = 0;
   Tensor slots;
+  require(kn.has_value() == vn.has_value() && kn.has_value() == slots_.has_value(),
+          "paged_prefill: new_kv must be (k, v, slots), each of them a tensor");
   if (kn) {
     require_device({&q, &*kn, &*vn, &*slots_});
     n_write = kn->size(0);

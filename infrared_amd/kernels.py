@@ -480,6 +480,8 @@ def paged_prefill(
             raise RuntimeError("paged_prefill: the plan was built for "
                                + ("fp32" if plan.f32 else "16-bit") + f" calls, q is {q.dtype}")
     kn, vn, slots = (None, None, None) if new_kv is None else new_kv
+    if new_kv is not None and kn is None:
+        raise RuntimeError("paged_prefill: new_kv must be (k, v, slots), each of them a tensor")
     return seam().paged_prefill(q, k_cache, v_cache, block_tables, cu_seqlens_q, q_start, int(max_q_len), block_size,
                                 scale, out, err_flags, None if plan is None else plan.buf, kn, vn, slots,
                                 int(src_row0), stream)

@@ -346,6 +346,21 @@ def test_native_calls_refuse_a_zero_block_size():
         kernels.paged_prefill(case.q, case.k_cache, case.v_cache, bt, cu, cl, 1, 0, 0.1)
 
 
+@pytest.mark.parametrize("missing", [(0,), (1,), (2,), (1, 2), (0, 1, 2)])
+def test_prefill_refuses_an_incomplete_new_kv(missing):
+    """new_kv = (k, v, slots) with any of them None is an error, not a read of nothing
+    and not a step whose write is left out."""
+    case = make_decode_case("qwen7b-bf16", DEV, num_seqs=2)
+    cu = torch.tensor([0, 1, 2], dtype=torch.int32, device=DEV)
+    rows = torch.zeros(2, 4, 128, dtype=torch.bfloat16, device=DEV)
+    new_kv = [rows, rows, torch.zeros(2, dtype=torch.int64, device=DEV)]
+    for i in missing:
+        new_kv[i] = None
+    with pytest.raises(RuntimeError, match="new_kv"):
+        kernels.paged_prefill(case.q, case.k_cache, case.v_cache, case.block_tables[0], cu, case.context_lens, 1, 16,
+                              0.1, new_kv=tuple(new_kv))
+
+
 def test_decode_one_hot_probe_returns_exact_v_row():
     """A key whose score dwarfs the rest makes the output equal its V row, which pins
     the block-table address of that key exactly."""
