@@ -66,6 +66,12 @@ void check_tables(const char* name, const Tensor& bt, const Tensor& ctx) {
   require(ctx.is_contiguous(), name, ": context_lens must be contiguous");
 }
 
+// A block size the C ABI's int holds (truncated it could divide by zero here).
+void check_block_size(const char* name, int64_t block_size) {
+  require(block_size > 0 && block_size <= INT32_MAX, name, "block_size must be positive and fit 32 bits, got ",
+          block_size);
+}
+
 void* ptr(const OptTensor& t) { return t ? t->data_ptr() : nullptr; }
 ir_stream_t stream_of(int64_t s) { return (ir_stream_t)(intptr_t)s; }
 
@@ -110,7 +116,7 @@ Tensor paged_decode(const Tensor& q, const Tensor& kc, const Tensor& vc, const T
   cache_layer("paged_decode", kc);
   check_tables("paged_decode", bt, ctx);
   require(q.dim() == 3, "paged_decode: q must be [B, H_q, D], got ", q.sizes());
-  require(block_size > 0, "paged_decode: block_size must be positive, got ", block_size);
+  check_block_size("paged_decode: ", block_size);
   const int b = (int)q.size(0), hq = (int)q.size(1), d = (int)q.size(2), h_kv = (int)kc.size(1);
   require(d == kc.size(2) && q.scalar_type() == kc.scalar_type() && vc.sizes() == kc.sizes(),
           "paged_decode: q / pool shape or dtype mismatch");
@@ -148,7 +154,7 @@ Tensor paged_decode_planned(const Tensor& q, const Tensor& kc, const Tensor& vc,
   cache_layer("paged_decode_planned", kc);
   require(q.dim() == 3, "paged_decode_planned: q must be [B, H_q, D], got ", q.sizes());
   const auto& [seqs, p_hq, p_hkv, max_blocks, bs, num_blocks, slot_stride, head_stride] = p;
-  require(bs > 0, "paged_decode_planned: the plan's block_size must be positive, got ", bs);
+  check_block_size("paged_decode_planned: the plan's ", bs);
   const int b = (int)q.size(0), hq = (int)q.size(1), d = (int)q.size(2);
   require(b == seqs && hq == p_hq && kc.size(1) == p_hkv, "paged_decode_planned: q / pool heads differ from the plan's");
   require(kc.size(0) / bs == num_blocks && kc.stride(0) == slot_stride && kc.stride(1) == head_stride &&
@@ -254,7 +260,7 @@ Tensor paged_prefill(const Tensor& q, const Tensor& kc, const Tensor& vc, const 
   require_device({&q, &kc, &vc, &bt, &cu, &q_start});
   cache_layer("paged_prefill", kc);
   require(q.dim() == 3, "paged_prefill: q must be [total_q, H_q, D], got ", q.sizes());
-  require(block_size > 0, "paged_prefill: block_size must be positive, got ", block_size);
+  check_block_size("paged_prefill: ", block_size);
   const int hq = (int)q.size(1), d = (int)q.size(2), h_kv = (int)kc.size(1);
   require(d == kc.size(2) && q.scalar_type() == kc.scalar_type() && vc.sizes() == kc.sizes(),
           "paged_prefill: q / pool shape or dtype mismatch");

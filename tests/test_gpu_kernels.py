@@ -335,15 +335,17 @@ def test_decode_flags_bad_block_ids_and_contexts():
     assert err.item() & ERR_CONTEXT_RANGE
 
 
-def test_native_calls_refuse_a_zero_block_size():
-    """A division in the native binding must not take the process down."""
+@pytest.mark.parametrize("block_size", [0, -16, 1 << 32])
+def test_native_calls_refuse_a_zero_block_size(block_size):
+    """A division in the native binding must not take the process down, nor by a size
+    that is zero in 32 bits."""
     case = make_decode_case("qwen7b-bf16", DEV, num_seqs=2)
     bt, cl = case.block_tables[0], case.context_lens
     with pytest.raises(RuntimeError, match="block_size"):
-        kernels.paged_decode(case.q, case.k_cache, case.v_cache, bt, cl, 0, 0.1)
+        kernels.paged_decode(case.q, case.k_cache, case.v_cache, bt, cl, block_size, 0.1)
     cu = torch.tensor([0, 1, 2], dtype=torch.int32, device=DEV)
     with pytest.raises(RuntimeError, match="block_size"):
-        kernels.paged_prefill(case.q, case.k_cache, case.v_cache, bt, cu, cl, 1, 0, 0.1)
+        kernels.paged_prefill(case.q, case.k_cache, case.v_cache, bt, cu, cl, 1, block_size, 0.1)
 
 
 @pytest.mark.parametrize("missing", [(0,), (1,), (2,), (1, 2), (0, 1, 2)])
