@@ -54,6 +54,8 @@ from infrared_amd import kernels
 from infrared_amd._lib import seam, stream_of
 from infrared_amd.paged_kv_cache import PagedKVPool
 
+_POOL_WRITE = PagedKVPool.write
+
 
 def paged_attention(
     q: torch.Tensor,
@@ -133,10 +135,14 @@ def _attend(q: torch.Tensor, paged, mask: torch.Tensor | None, layer_idx: int, s
         if new_kv is None:
             return
         k, v, slots = new_kv
-        if k.dim() != 4 or v.dim() != 4 or getattr(type(pool), "write", None) is not PagedKVPool.write or pool.strict:
+        # a write that is the pool's own, not a subclass's, the instance's or a wrapper
+        # put in its place (the class attribute may be patched too: compared with the
+        # function this module was loaded with), goes straight to the layer at hand
+        own = getattr(pool.write, "__func__", None) is _POOL_WRITE
+        if not own or k.dim() != 4 or v.dim() != 4 or pool.strict:
             h_kv, d = k.shape[-2:]
             pool.write(layer_idx, k.reshape(-1, h_kv, d), v.reshape(-1, h_kv, d), slots)
-        else:  # PagedKVPool.write on the layer already at hand
+        else:
             seam().write_step(k_layer, v_layer, k, v, slots, err, stream_of(k_layer))
 
     def rows():

@@ -968,3 +968,30 @@ def test_step_metadata_from_the_host_is_refused_under_capture():
             build_decode_static_inputs([[1]], [3], [7], 1, 32, 16, DEV, torch.float32)
     graph.replay()
     assert x.tolist() == [1.0] * 4  # the refusals left the capture whole
+
+
+@pytest.mark.parametrize("how", ["instance", "class", "subclass"])
+def test_a_replaced_pool_write_is_called(how, monkeypatch):
+    """A write put in the pool's place -- on the instance, on the class, in a subclass --
+    takes the step's K/V where the step is written before the attention."""
+    calls = []
+    own = PagedKVPool.write
+
+    def write(self, layer_idx, k, v, slots):
+        calls.append((layer_idx, tuple(k.shape)))
+        own(self, layer_idx, k, v, slots)
+
+    cls = type("Pool", (PagedKVPool,), {"write": write}) if how == "subclass" else PagedKVPool
+    if how == "class":
+        monkeypatch.setattr(PagedKVPool, "write", write)
+    pool = cls(2, 16, 16, 2, 64, torch.float32, device=DEV)
+    if how == "instance":
+        pool.write = lambda *args: write(pool, *args)
+    paged, mask = metadata.decode_context(pool, [[3], [4, 5]], [2, 20])
+    g = torch.Generator(device=DEV).manual_seed(1)
+    q, k, v = (torch.randn(2, 1, h, 64, generator=g, device=DEV) for h in (4, 2, 2))
+    paged_attention(q, k, v, paged, mask, 1, 0.125, 2)
+    paged.use_triton = False
+    paged_attention(q, k, v, paged, mask, 1, 0.125, 2)
+    assert calls == [(1, (2, 2, 64))] * 2
+    assert torch.equal(pool.k[1][paged.write_slots], k[:, 0])
