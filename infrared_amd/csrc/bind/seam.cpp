@@ -205,7 +205,13 @@ Tensor paged_attention_masked(const Tensor& q, const Tensor& kc, const Tensor& v
   if (h_kv > 0 && (!run_if || (int64_t)sq * (hq / h_kv) > 32)) {
     const int64_t need = ir_paged_attention_masked_workspace_size(b, sq, t, hq, h_kv, d, dtype_code(q), dtype_code(m),
                                                                   m.stride(3));
-    if (need > 0) ws = at::empty({need}, q.options().dtype(at::kByte));
+    if (need > 0) {
+      try {
+        ws = at::empty({need}, q.options().dtype(at::kByte));
+      } catch (const c10::OutOfMemoryError&) {
+        // a pool that leaves no room for it: one part, every tile, no workspace
+      }
+    }
   }
   check(ir_paged_attention_masked_ws(
             q.data_ptr(), q.stride(0), q.stride(1), q.stride(2), kc.data_ptr(), vc.data_ptr(), kc.stride(0),

@@ -12,7 +12,10 @@ import pytest
 import torch
 
 from infrared_amd import kernels, metadata
-from infrared_amd._lib import ERR_BLOCK_RANGE, ERR_CONTEXT_RANGE, ERR_GATHER_RANGE, ERR_SLOT_RANGE
+from infrared_amd._lib import (
+    DTYPE_BF16, ERR_BLOCK_RANGE, ERR_CONTEXT_RANGE, ERR_GATHER_RANGE, ERR_SLOT_RANGE, check, dtype_code, lib, ptr,
+    stream_ptr,
+)
 from infrared_amd.workloads import DECODE_CONFIGS, DecodeConfig, make_decode_case
 from oracle import naive as O
 
@@ -538,6 +541,46 @@ def test_masked_kernels_at_their_edges(b, sq, t, h_kv, n_rep, d, dtype, mask_dty
     assert bool((gated == 7.0).all())
 
 
+def _masked_without_workspace(q, kc, vc, gs, mask):
+    """ir_paged_attention_masked: no survey, every tile walked, one part."""
+    (b, sq, hq, d), (n, h_kv, _) = q.shape, kc.shape
+    out = torch.empty_like(q)
+    check(lib().ir_paged_attention_masked(
+        ptr(q), *q.stride()[:3], ptr(kc), ptr(vc), *kc.stride()[:2], n, ptr(gs), *gs.stride(), ptr(mask),
+        mask.stride(0), mask.stride(2), mask.stride(3), dtype_code(mask.dtype), ptr(out), *out.stride()[:3], b, sq,
+        gs.shape[1], hq, h_kv, d, d**-0.5, dtype_code(q.dtype), None, None, stream_ptr(q.device)),
+        "ir_paged_attention_masked")
+    return out
+
+
+def test_masked_runs_without_room_for_its_workspace():
+    """An allocator that has no room for a call's partial rows (a pool that takes all the
+    memory): the call runs in one part, as it does without a workspace."""
+    g = torch.Generator(device=DEV).manual_seed(2)
+    kc, vc = (torch.randn(4096, 4, 128, generator=g, device=DEV).bfloat16() for _ in range(2))
+    q = torch.randn(1, 512, 28, 128, generator=g, device=DEV).bfloat16()
+    gs = torch.randperm(4096, generator=g, device=DEV)[None]
+    mask = torch.zeros(1, 1, 512, 4096, dtype=torch.bfloat16, device=DEV)
+    need = lib().ir_paged_attention_masked_workspace_size(1, 512, 4096, 28, 4, 128, DTYPE_BF16, DTYPE_BF16, 1)
+    assert need > 0
+    want = _masked_without_workspace(q, kc, vc, gs, mask)
+    out = torch.empty_like(q)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (1 << 20)) / total)
+    try:
+        taken = []  # what the allocator still holds
+        with pytest.raises(torch.OutOfMemoryError):
+            while True:
+                taken.append(torch.empty(need, dtype=torch.uint8, device=DEV))
+        kernels.paged_attention_masked(q, kc, vc, gs, mask, 128**-0.5, out=out)
+        torch.cuda.synchronize()
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert torch.equal(out, want)
+
+
 @pytest.mark.parametrize("change", ["none", "row masked", "large scores", "nan in v", "inf in k", "bad slot", "faint bias"])
 @pytest.mark.parametrize("n_rep,d,dtype,lens", [
     (7, 128, torch.bfloat16, [(900, 1), (30, 40), (0, 129), (64, 64)]),
@@ -549,8 +592,6 @@ def test_masked_survey_leaves_out_only_what_adds_nothing(n_rep, d, dtype, lens, 
     values that are not finite, a slot outside the pool, a row that sees only a large
     negative bias. Held against the same call without a workspace (no survey, every
     tile walked) and, where the values are finite, the oracle."""
-    from infrared_amd._lib import check, dtype_code, lib, ptr, stream_ptr
-
     h_kv, slots_n = 2, 6000
     q_seq, q_pos, k_seq, k_pos = [], [], [], []
     for i, (start, n) in enumerate(lens):
@@ -587,12 +628,7 @@ def test_masked_survey_leaves_out_only_what_adds_nothing(n_rep, d, dtype, lens, 
     err = _err()
     out = kernels.paged_attention_masked(q, kc, vc, gs, mask, d**-0.5, err_flags=err)
     assert err.item() == (ERR_GATHER_RANGE if change == "bad slot" else 0)
-    dense = torch.empty_like(out)
-    check(lib().ir_paged_attention_masked_ws(
-        ptr(q), q.stride(0), q.stride(1), q.stride(2), ptr(kc), ptr(vc), kc.stride(0), kc.stride(1), kc.shape[0],
-        ptr(gs), gs.stride(0), gs.stride(1), ptr(mask), mask.stride(0), mask.stride(2), mask.stride(3),
-        dtype_code(dtype), ptr(dense), *dense.stride()[:3], 1, sq, t, h_kv * n_rep, h_kv, d, d**-0.5,
-        dtype_code(dtype), None, None, None, 0, stream_ptr(out.device)), "ir_paged_attention_masked_ws")
+    dense = _masked_without_workspace(q, kc, vc, gs, mask)
     assert torch.equal(out.isnan(), dense.isnan())
     # Each call rounds every probability to dtype (half an eps) relative to its own parts'
     # running maxima, so the two differ by at most eps * sum(p |v|) / sum(p) <= eps * max |v|,
