@@ -202,7 +202,7 @@ Tensor paged_attention_masked(const Tensor& q, const Tensor& kc, const Tensor& v
   }
   // a gated call of few columns takes its parts in one launch, without a workspace
   Tensor ws;
-  if (h_kv > 0 && (!run_if || (int64_t)sq * (hq / h_kv) > 32)) {
+  if (h_kv > 0 && (!run_if || (int64_t)sq * (hq / h_kv) > IR_MASKED_FEW_COLUMNS)) {
     const int64_t need = ir_paged_attention_masked_workspace_size(b, sq, t, hq, h_kv, d, dtype_code(q), dtype_code(m),
                                                                   m.stride(3));
     if (need > 0) {

@@ -870,12 +870,16 @@ struct Split {
 
 // The kernel a call takes and the parts it would use. The wide kernel needs a
 // 16-bit dtype, a mask of q's dtype or fp32 with unit key stride, and slots and
-// mask byte offsets that fit 32 bits.
+// mask byte offsets that fit 32 bits. Few columns fill little of a 128-column
+// workgroup: up to 16 the 16-column kernel is 1.2-1.5x faster (24 sequences x 2048
+// keys, 4 KV heads of 128, bf16, 14 columns: 24.8 us against 35.6 wide), 17 to 32
+// tie (28 columns: 40.6 / 36.8; one sequence of 4096: 14.1 / 17.1), and from 33 its
+// third pass over the keys loses (35 columns, 64 sequences x 2048: 137 / 75.8).
 Split split_of(int64_t batch, int64_t seq_q, int64_t seq_k, int num_q_heads, int num_kv_heads, int dtype,
                int mask_dtype, int64_t mask_t_stride, int64_t num_slots) {
   const int64_t rows = seq_q * (num_q_heads / num_kv_heads);
   Split s;
-  s.wide = rows > 32 && dtype != IR_DTYPE_F32 && (mask_dtype == dtype || mask_dtype == IR_DTYPE_F32) &&
+  s.wide = rows > IR_MASKED_FEW_COLUMNS && dtype != IR_DTYPE_F32 && (mask_dtype == dtype || mask_dtype == IR_DTYPE_F32) &&
            mask_t_stride == 1 && seq_k <= (1 << 28) && num_slots <= 0x7fffffff;
   // (the survey pays for itself from about 1000 keys; its bytes stay small)
   const int n_rep = num_q_heads / num_kv_heads;
