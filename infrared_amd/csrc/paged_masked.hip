@@ -276,6 +276,13 @@ constexpr float kScoreBound = 25e3f;  // 2 x this + kMasked - kClear stays far b
 constexpr int kSurveyTiles = 8;     // tiles of a mask workgroup: 8 keys a lane
 constexpr int kPartTiles = 6;       // tiles of a surveyed block worth a part of their own
 constexpr int kSurveyMin = 16;      // tiles from which a call is surveyed
+constexpr int64_t kSurveyMaxWgs = 1 << 24;  // a launch holds fewer than 2^32 threads
+
+// Workgroups of the survey: a tile of a KV head each, then kSurveyTiles tiles of a
+// column block's mask each (n_rtw blocks a sequence).
+inline int64_t survey_wgs(int64_t batch, int64_t num_kv_heads, int64_t nt, int64_t n_rtw) {
+  return batch * (num_kv_heads * nt + n_rtw * ((nt + kSurveyTiles - 1) / kSurveyTiles));
+}
 
 template <int DT, int D>
 __global__ __launch_bounds__(256) void paged_masked_survey_kernel(MaskedArgs a, int nt, int n_rtw) {
@@ -881,9 +888,12 @@ Split split_of(int64_t batch, int64_t seq_q, int64_t seq_k, int num_q_heads, int
   Split s;
   s.wide = rows > IR_MASKED_FEW_COLUMNS && dtype != IR_DTYPE_F32 && (mask_dtype == dtype || mask_dtype == IR_DTYPE_F32) &&
            mask_t_stride == 1 && seq_k <= (1 << 28) && num_slots <= 0x7fffffff;
-  // (the survey pays for itself from about 1000 keys; its bytes stay small)
+  // (the survey pays for itself from about 1000 keys; its bytes stay small, and
+  // its workgroups fit one launch)
   const int n_rep = num_q_heads / num_kv_heads;
-  s.survey = s.wide && mask_dtype == dtype && n_rep >= 5 && seq_k >= kSurveyMin * kTileKeys && seq_k <= (1 << 20);
+  const int64_t nt = (seq_k + kTileKeys - 1) / kTileKeys, n_rtw = (rows + kWideCols - 1) / kWideCols;
+  s.survey = s.wide && mask_dtype == dtype && n_rep >= 5 && seq_k >= kSurveyMin * kTileKeys && seq_k <= (1 << 20) &&
+             survey_wgs(batch, num_kv_heads, nt, n_rtw) < kSurveyMaxWgs;
   s.nwg = batch * num_kv_heads * (s.wide ? (rows + kWideCols - 1) / kWideCols : (rows + 15) / 16);
   const int64_t slots = (int64_t)device_cus() * 2;
   const int64_t units = s.wide ? (seq_k + kTileKeys - 1) / kTileKeys / 2 : (seq_k + 15) / 16 / (2 * kWaves);
@@ -920,8 +930,8 @@ void launch(const MaskedArgs& a, const Split& sp, hipStream_t s) {
       else if (a.n_rep >= 5) {
         if (a.vis) {
           const int nt = (a.seq_k + kTileKeys - 1) / kTileKeys, n_rtw = (int)(sp.nwg / a.num_kv_heads / a.batch);
-          const int64_t wgs = (int64_t)a.batch * (a.num_kv_heads * nt + n_rtw * ((nt + kSurveyTiles - 1) / kSurveyTiles));
-          hipLaunchKernelGGL((paged_masked_survey_kernel<DT, D>), dim3((unsigned)wgs), dim3(256), 0, s, a, nt, n_rtw);
+          const unsigned wgs = (unsigned)survey_wgs(a.batch, a.num_kv_heads, nt, n_rtw);
+          hipLaunchKernelGGL((paged_masked_survey_kernel<DT, D>), dim3(wgs), dim3(256), 0, s, a, nt, n_rtw);
           hipLaunchKernelGGL((paged_masked_walks_kernel<DT, D>), dim3((unsigned)sp.nwg), dim3(256), 0, s, a, nt, n_rtw);
         }
         hipLaunchKernelGGL((paged_masked_wide_kernel<DT, D, 2, true>), grid, block, 0, s, a);

@@ -147,6 +147,16 @@ def _plan_bytes(num_seqs, max_q, n_rep, h_kv, d, cus=256, xcds=1, cols=128):
     return a(entries * 8) + a(cap * h_kv * 4) + a(rows * 8) + a(rows * d * 4)
 
 
+def test_masked_workspace_covers_a_survey_only_where_one_launch_holds_it():
+    """512 sequences x 65536 keys x 32 KV heads are 2^24 key tiles, a workgroup of 256
+    threads each: more than a launch holds, so no survey and, the device being full, no
+    workspace at all. Half as many sequences are surveyed."""
+    size = _lib.lib().ir_paged_attention_masked_workspace_size
+    args = (256, 65536, 224, 32, 128, _lib.DTYPE_BF16, _lib.DTYPE_BF16, 1)
+    assert size(512, *args) == 0
+    assert size(250, *args) > 250 * 32 * 1024 * 4  # at least a bound per key tile and KV head
+
+
 def test_prefill_plan_helpers():
     """A prefill plan's size follows its documented layout (8 or 2 chunks of
     512 tokens at 28 / 4 heads: 29 blocks of 18 tokens each, two workgroups per
