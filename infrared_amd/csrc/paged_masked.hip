@@ -274,8 +274,10 @@ constexpr float kMasked = -6e4f;    // fp16's finfo.min is -65504
 constexpr float kClear = -1e3f;
 constexpr float kScoreBound = 25e3f;  // 2 x this + kMasked - kClear stays far below any exponent
 constexpr int kSurveyTiles = 8;     // tiles of a mask workgroup: 8 keys a lane
-constexpr int kPartTiles = 6;       // tiles of a surveyed block worth a part of their own
-constexpr int kSurveyMin = 16;      // tiles from which a call is surveyed
+constexpr int kPartTiles = 6;       // tiles of a surveyed block worth a part of their own (12: 72 us against 60
+                                    // on 5 decodes and 3 chunks of 170, 79 against 87 on 3 chunks of 180 after 2000)
+constexpr int kSurveyMin = 16;      // a surveyed call has at least these tiles
+constexpr int kSurveyBlocks = 12;   // and 128-column blocks per (sequence, KV head)
 constexpr int64_t kSurveyMaxWgs = 1 << 24;  // a launch holds fewer than 2^32 threads
 
 // Workgroups of the survey: a tile of a KV head each, then kSurveyTiles tiles of a
@@ -882,23 +884,38 @@ struct Split {
 // keys, 4 KV heads of 128, bf16, 14 columns: 24.8 us against 35.6 wide), 17 to 32
 // tie (28 columns: 40.6 / 36.8; one sequence of 4096: 14.1 / 17.1), and from 33 its
 // third pass over the keys loses (35 columns, 64 sequences x 2048: 137 / 75.8).
-Split split_of(int64_t batch, int64_t seq_q, int64_t seq_k, int num_q_heads, int num_kv_heads, int dtype,
-               int mask_dtype, int64_t mask_t_stride, int64_t num_slots) {
-  const int64_t rows = seq_q * (num_q_heads / num_kv_heads);
-  Split s;
-  s.wide = rows > IR_MASKED_FEW_COLUMNS && dtype != IR_DTYPE_F32 && (mask_dtype == dtype || mask_dtype == IR_DTYPE_F32) &&
-           mask_t_stride == 1 && seq_k <= (1 << 28) && num_slots <= 0x7fffffff;
-  // (the survey pays for itself from about 1000 keys; its bytes stay small, and
-  // its workgroups fit one launch)
+Split split_of(int64_t batch, int64_t seq_q, int64_t seq_k, int num_q_heads, int num_kv_heads, int head_dim,
+               int dtype, int mask_dtype, int64_t mask_t_stride, int64_t num_slots) {
   const int n_rep = num_q_heads / num_kv_heads;
+  const int64_t rows = seq_q * n_rep;
+  Split s;
+  s.wide = rows > IR_MASKED_FEW_COLUMNS && dtype != IR_DTYPE_F32 &&
+           (mask_dtype == dtype || mask_dtype == IR_DTYPE_F32) && mask_t_stride == 1 && seq_k <= (1 << 28) &&
+           num_slots <= 0x7fffffff;
   const int64_t nt = (seq_k + kTileKeys - 1) / kTileKeys, n_rtw = (rows + kWideCols - 1) / kWideCols;
-  s.survey = s.wide && mask_dtype == dtype && n_rep >= 5 && seq_k >= kSurveyMin * kTileKeys && seq_k <= (1 << 20) &&
-             survey_wgs(batch, num_kv_heads, nt, n_rtw) < kSurveyMaxWgs;
-  s.nwg = batch * num_kv_heads * (s.wide ? (rows + kWideCols - 1) / kWideCols : (rows + 15) / 16);
   const int64_t slots = (int64_t)device_cus() * 2;
-  const int64_t units = s.wide ? (seq_k + kTileKeys - 1) / kTileKeys / 2 : (seq_k + 15) / 16 / (2 * kWaves);
+  s.nwg = batch * num_kv_heads * (s.wide ? n_rtw : (rows + 15) / 16);
+  // The survey reads all keys and the mask once, a launch of ~10 us or one column
+  // block's walk, whichever is more, and the walks another ~8: it can pay where
+  // several blocks walk the same keys, long enough. bf16, 4 KV heads of 128, with
+  // it against without: 256 tokens in 4 chunks after 2000 keys each (14 blocks, 131
+  // tiles) 60 / 76 us, after 500 (37 tiles) 45 / 39; 512 in 8 after 200 (28, 39) 46 /
+  // 54; 1024 in 16 (56, 291) 101 / 522; a 2048-token prompt (112, 32) 118 / 127. Few
+  // blocks lose at any length: 73 tokens, 13 of them decodes (4, 257) 70 / 51; 64
+  // sequences x 5 tokens (1, 32) 137 / 76. Tiles of 64 channels take less time each, so
+  // more of them (2 KV heads: 515 tokens, 29 blocks, 101 tiles 41 / 45; 305, 17, 98 37 /
+  // 33). A dense frame loses what the survey costs (512 tokens at the end of 4096 keys:
+  // 108 / 78), which sizes alone do not tell.
+  const bool worth = n_rtw >= kSurveyBlocks && nt >= kSurveyMin && s.nwg * nt >= slots * (head_dim == 64 ? 11 : 8);
+  // (seq_k: its bytes stay small; its workgroups fit one launch)
+  s.survey = s.wide && worth && mask_dtype == dtype && n_rep >= 5 && seq_k <= (1 << 20) &&
+             survey_wgs(batch, num_kv_heads, nt, n_rtw) < kSurveyMaxWgs;
+  const int64_t units = s.wide ? nt / 2 : (seq_k + 15) / 16 / (2 * kWaves);
   s.parts = (int)std::max<int64_t>(1, std::min<int64_t>({s.nwg > 0 ? slots / s.nwg : 1, units, 64}));
-  // surveyed walks differ in length; parts beyond a block's own need cost nothing
+  // Surveyed walks differ in length: a block that holds decode rows walks all their
+  // histories. More parts than fill the device cut it (13 decodes and 4 chunks after
+  // 1000 keys: 178 us against 473 without them; 5 decodes and 3 chunks 60 / 98), and
+  // cost a dense frame their merge (512 tokens after 3584: 107 / 89).
   if (s.survey && s.nwg < 2 * slots) s.parts = std::max(s.parts, (int)std::min<int64_t>(units, kSurveyParts));
   return s;
 }
@@ -962,7 +979,8 @@ extern "C" int64_t ir_paged_attention_masked_workspace_size(int batch, int seq_q
   if (batch <= 0 || seq_q <= 0 || seq_k <= 0 || num_q_heads <= 0 || num_kv_heads <= 0 ||
       num_q_heads % num_kv_heads != 0 || (head_dim != 64 && head_dim != 128))
     return 0;
-  const Split sp = split_of(batch, seq_q, seq_k, num_q_heads, num_kv_heads, dtype, mask_dtype, mask_t_stride, 0);
+  const Split sp = split_of(batch, seq_q, seq_k, num_q_heads, num_kv_heads, head_dim, dtype, mask_dtype,
+                            mask_t_stride, 0);
   const int64_t per = part_bytes(batch, seq_q, num_q_heads, head_dim);
   const int64_t parts = std::min<int64_t>(sp.parts, kMaxPartBytes / per);
   return (parts > 1 ? parts * per : 0) + survey_bytes(sp, batch, seq_k, num_kv_heads).total();
@@ -1049,8 +1067,8 @@ extern "C" int ir_paged_attention_masked_ws(const void* q, int64_t q_b_stride, i
   a.scale = scale;
   a.err = err_flags;
   a.run_if = run_if;
-  const Split sp = split_of(batch, seq_q, seq_k, a.num_q_heads, num_kv_heads, dtype, mask_dtype, mask_t_stride,
-                            num_slots);
+  const Split sp = split_of(batch, seq_q, seq_k, a.num_q_heads, num_kv_heads, head_dim, dtype, mask_dtype,
+                            mask_t_stride, num_slots);
   // as many parts as pay and the workspace holds (none: one part)
   const int64_t per = part_bytes(batch, seq_q, num_q_heads, head_dim);
   IR_REQUIRE(workspace_bytes >= 0 && (!workspace || aligned16(workspace)),

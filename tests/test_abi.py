@@ -157,6 +157,31 @@ def test_masked_workspace_covers_a_survey_only_where_one_launch_holds_it():
     assert size(250, *args) > 250 * 32 * 1024 * 4  # at least a bound per key tile and KV head
 
 
+def test_masked_survey_needs_blocks_and_tiles():
+    """A surveyed call has 12 blocks of 128 columns a sequence, and 8 key tiles (11 at
+    head_dim 64) for each of the 512 workgroups the device holds: the workspace on both
+    sides of each line, as the parts' fp32 rows and the survey's four regions."""
+    size = _lib.lib().ir_paged_attention_masked_workspace_size
+    up = lambda x: (x + 255) // 256 * 256  # noqa: E731
+    kv, heads = 4, 8  # KV heads, query heads of each: 16 tokens a block
+
+    def want(blocks, nt, d, surveyed):
+        nwg = blocks * kv
+        parts = min(512 // nwg, nt // 2)
+        regions = 0
+        if surveyed:
+            parts = max(parts, min(nt // 2, 12))
+            regions = up(blocks * up(nt * 4) // 4) + up(blocks * -(-nt // 8) * 32) + up(nwg * 8) + up(kv * nt * 4)
+        return parts * blocks * 16 * kv * heads * (d + 2) * 4 + regions
+
+    def got(blocks, nt, d):
+        return size(1, blocks * 16, nt * 64, kv * heads, kv, d, _lib.DTYPE_BF16, _lib.DTYPE_BF16, 1)
+
+    for blocks, nt, d, surveyed in ((12, 86, 128, True), (12, 85, 128, False), (12, 118, 64, True),
+                                    (12, 117, 64, False), (11, 200, 128, False), (11, 200, 64, False)):
+        assert got(blocks, nt, d) == want(blocks, nt, d, surveyed), (blocks, nt, d)
+
+
 def test_prefill_plan_helpers():
     """A prefill plan's size follows its documented layout (8 or 2 chunks of
     512 tokens at 28 / 4 heads: 29 blocks of 18 tokens each, two workgroups per

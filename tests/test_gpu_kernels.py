@@ -497,7 +497,8 @@ def test_masked_fully_masked_row_is_uniform_and_bad_slot_flagged():
     (1, 130, 200, 1, 1, 64, torch.float16, torch.float16),    # one head a token
     (1, 27, 130, 1, 5, 128, torch.bfloat16, torch.bfloat16),  # 5 heads: 27 tokens in a workgroup
     (1, 9, 4200, 1, 40, 64, torch.bfloat16, torch.bfloat16),  # 40 heads a token
-    (2, 40, 1100, 2, 7, 128, torch.float16, torch.float16),   # two sequences, surveyed
+    (2, 40, 1100, 2, 7, 128, torch.float16, torch.float16),   # two sequences
+    (2, 250, 1100, 10, 7, 128, torch.float16, torch.float16), # two sequences, surveyed
 ])
 @pytest.mark.parametrize("strided", [False, True])
 def test_masked_kernels_at_their_edges(b, sq, t, h_kv, n_rep, d, dtype, mask_dtype, strided):
@@ -583,8 +584,8 @@ def test_masked_runs_without_room_for_its_workspace():
 
 @pytest.mark.parametrize("change", ["none", "row masked", "large scores", "nan in v", "inf in k", "bad slot", "faint bias"])
 @pytest.mark.parametrize("n_rep,d,dtype,lens", [
-    (7, 128, torch.bfloat16, [(900, 1), (30, 40), (0, 129), (64, 64)]),
-    (7, 64, torch.float16, [(0, 64), (4100, 3), (64, 20)]),
+    (7, 128, torch.bfloat16, [(2900, 1), (30, 40), (0, 129), (64, 64)]),
+    (7, 64, torch.float16, [(0, 64), (4100, 3), (64, 150)]),
 ])
 def test_masked_survey_leaves_out_only_what_adds_nothing(n_rep, d, dtype, lens, change):
     """A long packed frame with the block-diagonal varlen mask, and every reason not to
@@ -592,7 +593,7 @@ def test_masked_survey_leaves_out_only_what_adds_nothing(n_rep, d, dtype, lens, 
     values that are not finite, a slot outside the pool, a row that sees only a large
     negative bias. Held against the same call without a workspace (no survey, every
     tile walked) and, where the values are finite, the oracle."""
-    h_kv, slots_n = 2, 6000
+    h_kv, slots_n = 9, 6000
     q_seq, q_pos, k_seq, k_pos = [], [], [], []
     for i, (start, n) in enumerate(lens):
         q_seq += [i] * n
