@@ -8,6 +8,7 @@ missing or a call fails, a ``RuntimeError`` names the cause.
 
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import os
 import threading
@@ -183,6 +184,12 @@ def stream_of(t: torch.Tensor) -> int:
     if _raw_stream is None:
         return stream_ptr(t.device)
     return _raw_stream(t.get_device())
+
+
+def on_device(device: torch.device):
+    """Context in which a call launches on ``device``, whichever is current (its
+    stream's raw handle may be the null stream, which is the current device's)."""
+    return torch.cuda.device(device) if device.type == "cuda" else contextlib.nullcontext()
 
 
 def check(rc: int, what: str) -> None:

@@ -31,7 +31,7 @@ import numpy as np
 import torch
 
 from infrared_amd import metadata
-from infrared_amd._lib import check, dtype_code, lib, ptr, stream_ptr
+from infrared_amd._lib import check, dtype_code, lib, on_device, ptr, stream_ptr
 from infrared_amd.paged_kv_cache import PagedContext, PagedKVPool, host_list, to_device
 
 
@@ -157,11 +157,12 @@ def _fill_inputs(out: DecodeInputs, block_tables: Sequence[Sequence[int]], num_c
     metadata.fill_tables(host[4 * b :].reshape(b, width), [list(block_tables[j])[:width] for j in range(b)])
     dev = out.mask.device
     staging = to_device(host, dev)
-    check(lib().ir_decode_inputs(
-        ptr(staging), b, bucket_b, width, block_size, out.mask.shape[-1], dtype_code(out.mask.dtype), ptr(out.ids),
-        ptr(out.positions), ptr(out.write_slots), ptr(out.gather_slots), ptr(out.mask), ptr(out.block_tables),
-        ptr(out.context_lens), stream_ptr(dev),
-    ), "ir_decode_inputs")
+    with on_device(dev):
+        check(lib().ir_decode_inputs(
+            ptr(staging), b, bucket_b, width, block_size, out.mask.shape[-1], dtype_code(out.mask.dtype), ptr(out.ids),
+            ptr(out.positions), ptr(out.write_slots), ptr(out.gather_slots), ptr(out.mask), ptr(out.block_tables),
+            ptr(out.context_lens), stream_ptr(dev),
+        ), "ir_decode_inputs")
     # written through raw pointers: what is cached of these tensors (the pool's
     # reference-form check of gather_slots and mask) has to see that they changed
     torch.autograd.graph.increment_version([getattr(out, n) for n in DecodeInputs.__slots__])

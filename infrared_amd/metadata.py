@@ -25,7 +25,7 @@ from operator import index
 import numpy as np
 import torch
 
-from infrared_amd._lib import check, lib, ptr, stream_ptr
+from infrared_amd._lib import check, lib, on_device, ptr, stream_ptr
 from infrared_amd.paged_kv_cache import PagedContext, PagedKVPool, host_list, row_split, to_device
 
 
@@ -182,9 +182,10 @@ def prefill_context(
     bt = flat[: n * width].view(n, width)
     nc, cu = flat[n * width : n * width + n], flat[n * width + n :]
     write_slots = torch.empty(total, dtype=torch.int64, device=flat.device)
-    check(lib().ir_packed_write_slots(
-        ptr(bt), width, width, ptr(nc), ptr(cu), n, total, bs, ptr(write_slots), stream_ptr(flat.device),
-    ), "ir_packed_write_slots")
+    with on_device(flat.device):
+        check(lib().ir_packed_write_slots(
+            ptr(bt), width, width, ptr(nc), ptr(cu), n, total, bs, ptr(write_slots), stream_ptr(flat.device),
+        ), "ir_packed_write_slots")
     ctx = PagedContext(pool, write_slots, None, use_triton, bt, None, cu, nc, max(q_lens, default=0))
     ctx.row_split = row_split(bt, num_cached, q_lens)
     if not with_mask:

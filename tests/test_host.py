@@ -4,6 +4,8 @@ and the oracle's loop restatements."""
 
 from __future__ import annotations
 
+import contextlib
+
 import numpy as np
 import pytest
 import torch
@@ -257,3 +259,37 @@ def test_host_metadata_is_refused_under_capture(monkeypatch):
     with pytest.raises(RuntimeError, match="capturing"):
         paged_kv_cache.to_device(np.zeros(4, dtype=np.int32), "cuda")
     assert paged_kv_cache.to_device(np.arange(3), "cpu").tolist() == [0, 1, 2]
+
+
+@pytest.mark.parametrize("call", ["decode", "prefill"])
+def test_step_metadata_is_built_on_its_own_device(call, monkeypatch):
+    """The two metadata launches run with their tensors' device current, as the library
+    calls they replaced did by themselves."""
+    current = []
+
+    @contextlib.contextmanager
+    def on_device(device):
+        current.append(device)
+        yield
+        current.pop()
+
+    calls = []
+
+    class Recorder:
+        def ir_decode_inputs(self, *args):
+            calls.append(list(current))
+            return 0
+
+        ir_packed_write_slots = ir_decode_inputs
+
+    cpu = torch.device("cpu")
+    for module in (hip_graph, metadata):
+        monkeypatch.setattr(module, "lib", Recorder)
+        monkeypatch.setattr(module, "on_device", on_device)
+        monkeypatch.setattr(module, "stream_ptr", lambda device: 0)
+    if call == "decode":
+        buf = hip_graph.build_decode_static_inputs([[1]], [3], [7], 1, 32, 16, cpu, torch.float32)
+        hip_graph._fill_inputs(buf, [[1]], [3], [7], 16)
+    else:
+        metadata.prefill_context(type("Pool", (), {"device": cpu, "block_size": 16})(), [[1]], [3], [2])
+    assert calls == [[cpu]] and not current
