@@ -613,16 +613,28 @@ def test_masked_survey_leaves_out_only_what_adds_nothing(n_rep, d, dtype, lens, 
     elif change == "large scores":
         q *= 3000.0
         kc *= 40.0
+        mask[mask < -6e4] = -61440.0  # (finfo(bf16).min would drown any score)
     elif change == "nan in v":
         vc[gs[0, 5]] = float("nan")
     elif change == "inf in k":
         kc[gs[0, 5], :, 3] = float("inf")
     elif change == "faint bias":
-        mask[0, 0, sq // 2] = torch.finfo(dtype).min
+        # q.k * scale is 19.9e3, and -19.9e3 for the one key the row sees at -5e4: its
+        # masked keys, at -65504 or so, come out ahead of it
+        c, e = (32.0, 55.0) if d == 128 else (40.0, 62.0)
+        q.fill_(c)
+        kc.fill_(e)
+        kc[gs[0, t // 2]] = -e
+        mask[0, 0, sq // 2] = max(torch.finfo(dtype).min, -65536.0)
         mask[0, 0, sq // 2, t // 2] = -5e4
     ref = None
+    naive = lambda m: O.paged_attention_naive(q.float(), kc.float(), vc.float(), gs, m, d**-0.5, n_rep)  # noqa: E731
     if change in ("none", "row masked", "faint bias"):
-        ref = O.paged_attention_naive(q.float(), kc.float(), vc.float(), gs, mask.float(), d**-0.5, n_rep)
+        ref = naive(mask.float())
+    if change in ("large scores", "faint bias"):
+        # leaving out every tile nothing is visible in would show
+        blind = mask.float().masked_fill(mask <= -6e4, float("-inf"))
+        assert (naive(blind) - naive(mask.float())).abs().max().item() > 10 * TOL[dtype]
     if change == "bad slot":
         gs[0, 7] = slots_n
     q, kc, vc, gs, mask = (x.to(DEV) for x in (q, kc, vc, gs, mask))
@@ -641,6 +653,98 @@ def test_masked_survey_leaves_out_only_what_adds_nothing(n_rep, d, dtype, lens, 
         assert bool(out.isnan().any())
     if ref is not None:
         assert (out.float().cpu() - ref).abs().max().item() <= TOL[dtype]
+
+
+def _survey_regions(blocks, h_kv, b, nt):
+    """Byte offsets of walks and of the end of a surveyed call's workspace head, as the
+    survey lays it out: tiles seen per column block, tokens seen per group of 8 tiles,
+    then (parts, tiles) per (sequence, KV head, block), then a bound per key tile."""
+    up = lambda x: (x + 255) // 256 * 256  # noqa: E731
+    walks = up(b * blocks * (-(-nt // 64) * 64)) + up(b * blocks * -(-nt // 8) * 32)
+    return walks, walks + up(b * h_kv * blocks * 8) + up(b * h_kv * nt * 4)
+
+
+@pytest.mark.parametrize("room", ["full", "survey only", "two parts"])
+def test_masked_survey_per_sequence_and_head(room):
+    """Three frames in one call, each with its own block-diagonal mask; one KV head of the
+    second has a NaN in V, so that head walks every tile there and the rest skip. The
+    walks, read back from a workspace of the caller's, are those the masks ask for; the
+    outputs are the unsurveyed call's and the oracle's; a gated call gives the same bits,
+    and with a workspace that holds fewer parts, or none beside the survey, so do the walks."""
+    b, sq, t, h_kv, n_rep, d, dtype = 3, 217, 2200, 4, 7, 128, torch.bfloat16
+    frames = [[(900, 100), (1000, 100), (83, 17)], [(1900, 60), (83, 157)], [(100, 17), (1783, 100), (100, 100)]]
+    g = torch.Generator().manual_seed(17)
+    masks = []
+    for lens in frames:
+        assert (sum(n for _, n in lens), sum(s + n for s, n in lens)) == (sq, t)
+        ids = [torch.tensor(x) for x in (
+            [i for i, (s, n) in enumerate(lens) for _ in range(n)], [s + j for s, n in lens for j in range(n)],
+            [i for i, (s, n) in enumerate(lens) for _ in range(s + n)], [p for s, n in lens for p in range(s + n)])]
+        masks.append(O.varlen_mask(*ids, dtype))
+    mask = torch.cat(masks)
+    gs = torch.randperm(b * t, generator=g).view(b, t)
+    kc, vc = (torch.randn(b * t, h_kv, d, generator=g).to(dtype) for _ in range(2))
+    q = torch.randn(b, sq, h_kv * n_rep, d, generator=g).to(dtype)
+    ref = O.paged_attention_naive(q.float(), kc.float(), vc.float(), gs, mask.float(), d**-0.5, n_rep)
+    nan_head = slice(2 * n_rep, 3 * n_rep)
+    vc[gs[1, 5], 2] = float("nan")
+
+    blocks, nt = -(-sq * n_rep // 128), -(-t // 64)
+    seen = torch.zeros(b, sq, nt * 64, dtype=torch.bool)
+    seen[..., :t] = mask[:, 0] > -6e4
+    seen = seen.view(b, sq, nt, 64).any(-1)
+    tiles = torch.stack([seen[:, i * 128 // n_rep : min(i * 128 + 127, sq * n_rep - 1) // n_rep + 1].any(1).sum(1)
+                         for i in range(blocks)], 1)  # [b, blocks]
+    assert int(tiles.min()) < nt // 2  # there is something to leave out
+    tiles = tiles[:, None].expand(b, h_kv, blocks).clone()
+    tiles[1, 2] = nt
+
+    q, kc, vc, gs, mask = (x.to(DEV) for x in (q, kc, vc, gs, mask))
+    walks_at, survey_end = _survey_regions(blocks, h_kv, b, nt)
+    code = dtype_code(dtype)
+    need = lib().ir_paged_attention_masked_workspace_size(b, sq, t, h_kv * n_rep, h_kv, d, code, code, 1)
+    part = b * sq * h_kv * n_rep * (d + 2) * 4
+    parts = (need - survey_end) // part
+    assert need == survey_end + parts * part and parts > 2
+    if room != "full":
+        parts = 1 if room == "survey only" else 2
+        need = survey_end + (0 if parts == 1 else parts * part)
+    err = _err()
+
+    def call(run_if=None, out=None):
+        out = torch.empty_like(q) if out is None else out
+        ws = torch.zeros(need, dtype=torch.uint8, device=DEV)
+        check(lib().ir_paged_attention_masked_ws(
+            ptr(q), *q.stride()[:3], ptr(kc), ptr(vc), *kc.stride()[:2], kc.shape[0], ptr(gs), *gs.stride(), ptr(mask),
+            mask.stride(0), mask.stride(2), mask.stride(3), code, ptr(out), *out.stride()[:3], b, sq, t,
+            h_kv * n_rep, h_kv, d, d**-0.5, code, ptr(err), ptr(run_if), ptr(ws), need, stream_ptr(q.device)),
+            "ir_paged_attention_masked_ws")
+        return out, ws[walks_at : walks_at + b * h_kv * blocks * 8].view(torch.int32).view(b, h_kv, blocks, 2).cpu()
+
+    out, walks = call()
+    want = torch.stack([torch.clamp((tiles + 5) // 6, max=parts), tiles], -1)
+    want[1, 2, :, 0] *= -1  # parts < 0: a walk of all tiles
+    assert torch.equal(walks, want.int())
+    assert err.item() == 0
+    dense = _masked_without_workspace(q, kc, vc, gs, mask)
+    assert torch.equal(out.isnan(), dense.isnan())
+    assert bool(out[1, :, nan_head].isnan().all()) and not out[[0, 2]].isnan().any()
+    # (the bound of the test above: probabilities rounded against other running maxima)
+    eps = torch.finfo(dtype).eps
+    vmax = vc[vc.isfinite()].abs().max().item()
+    assert torch.allclose(out.float(), dense.float(), rtol=eps, atol=eps * vmax, equal_nan=True)
+    diff = (out.float().cpu() - ref).abs()
+    diff[1, :, nan_head] = 0.0
+    assert diff.max().item() <= TOL[dtype]
+    if room == "full":
+        got = kernels.paged_attention_masked(q, kc, vc, gs, mask, d**-0.5)
+        assert torch.equal(got.nan_to_num(7.0), out.nan_to_num(7.0))
+    gate = torch.ones(1, dtype=torch.int32, device=DEV)
+    gated, gated_walks = call(gate)
+    assert torch.equal(gated.nan_to_num(7.0), out.nan_to_num(7.0)) and torch.equal(gated_walks, walks)
+    gate.zero_()
+    untouched, _ = call(gate, torch.full_like(out, 3.0))
+    assert bool((untouched == 3.0).all())
 
 
 def test_config_table_is_consistent():
