@@ -264,12 +264,13 @@ void paged_masked_kernel(MaskedArgs a) {
 // a 128-column block may see, and what they add is exactly zero -- provided every
 // row sees some key clearly, no score is large enough to bring a masked key back,
 // and V is finite (0 * inf is NaN). This kernel finds out, so that the wide
-// kernel may leave those tiles out with the same result bit by bit: per (KV head,
-// tile) the largest |K|, and per (column block, tile) whether any mask value is
-// above kMasked, with a flag for each token that has one above kClear. One pass
-// over the mask and the frame's keys. 610 tokens x 5333 keys (8 sequences),
-// 28/4 heads of 128, bf16: 9 us + 7.5 us for the walks, after which the wide kernel
-// takes 35 us instead of 109.
+// kernel may leave those tiles out; its parts are then cut from the tiles that
+// remain, so probabilities are rounded against other running maxima than without
+// a survey. It finds per (KV head, tile) the largest |K|, and per (column block,
+// tile) whether any mask value is above kMasked, with a flag for each token that
+// has one above kClear. One pass over the mask and the frame's keys. 610 tokens x
+// 5333 keys (8 sequences), 28/4 heads of 128, bf16: 9 us + 7.5 us for the walks,
+// after which the wide kernel takes 35 us instead of 109.
 constexpr float kMasked = -6e4f;    // fp16's finfo.min is -65504
 constexpr float kClear = -1e3f;
 constexpr float kScoreBound = 25e3f;  // 2 x this + kMasked - kClear stays far below any exponent
@@ -449,12 +450,14 @@ __global__ __launch_bounds__(256) void paged_masked_walks_kernel(MaskedArgs a, i
 // row-major with 32 bytes of padding a row (conflict-free operand reads; V^T
 // through the transpose read), in a 2-deep ring: tile kb is computed while tile
 // kb + 1 goes from registers to the other buffer, tile kb + 2's K and V and
-// tile kb + 3's slots are in flight. Two workgroups share a CU (74 KB of LDS,
-// at most 256 registers). 610 tokens x 5333 keys, 28/4 heads of 128, bf16: 109 + 7.5
-// us (merge; 420 TFLOP/s over all pairs, masked ones included) against 827 us with
-// 16 columns a workgroup and no staging: there every 16 columns read all keys
-// again. The matrix and vector pipes carry the rest about equally, as in the
-// chunked prefill.
+// tile kb + 3's slots are in flight. Two workgroups share a CU (at most 256
+// registers; at head_dim 128 81,712 B of LDS with a staged mask, 208 B below half of
+// a CU's, 74,384 B without). 610 tokens x 5333 keys, 28/4 heads of 128, bf16: 109 +
+// 7.5 us (merge; 420 TFLOP/s over all pairs, masked ones included) against 827 us with
+// 16 columns a workgroup and no staging: there every 16 columns read all keys again.
+// Bound by the vector pipe's issue and by latency: 8 vector instructions a MFMA, 2.0
+// times the matrix pipe's busy cycles, 43% of wavefront time in waits, 21% waiting to
+// issue, no LDS bank conflicts (the same frame, surveyed).
 //
 // MB: bytes of a mask element (2: the dtype of q; 4: fp32). ML: the mask tile goes
 // through LDS too, loaded a tile ahead once per token instead of once per column
@@ -476,6 +479,8 @@ void paged_masked_wide_kernel(MaskedArgs a) {
   __shared__ __attribute__((aligned(16))) uint16_t mk_lds[ML ? 2 : 1][ML ? kMaskTokens * MP : 8];
   __shared__ int slot_lds[2][BN];
   __shared__ uint8_t key_ok[2][BN];
+  static_assert(sizeof(ks_lds) + sizeof(vs_lds) + sizeof(mk_lds) + sizeof(slot_lds) + sizeof(key_ok) <= 80 * 1024,
+                "two workgroups per CU");
   static_assert(!ML || (MB == 2 && kMaskTokens * (BN / 4) <= 2 * NT), "two 4-key mask pieces a thread");
   if (a.run_if && *a.run_if == 0) return;
 

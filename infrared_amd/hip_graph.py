@@ -229,7 +229,7 @@ class HipGraphDecoder:
                 block_tables, num_cached, last_tokens, bucket, self.t_max, self.block_size,
                 self.device, self.dtype,
             )
-            if bucket in self._graphs:
+            if bucket in self._graphs:  # (a dtype or bucket the kernel does not take)
                 self._copy_inputs(self._graphs[bucket].buf, inp)
             else:
                 self._capture(bucket, inp)

@@ -69,7 +69,9 @@ def packed_write_slots(
     """``[sum(q_lens)]`` int64 slots of a packed step's new tokens, in packing
     order: sequence ``b``'s ``q_lens[b]`` tokens at positions ``num_cached[b] ..``
     map to ``slot(bt_b, p) = bt_b[p // bs] * bs + p % bs``
-    (``infrared/engine/paged_engine.py:621-625``), computed on the tables' device."""
+    (``infrared/engine/paged_engine.py:621-625``), computed on the tables' device
+    with library operations: for tables and lengths that are there already
+    (``prefill_context`` takes host lists and runs ``ir_packed_write_slots``)."""
     dev = block_tables.device
     q_lens = q_lens.to(device=dev, dtype=torch.long)
     nc = num_cached.to(device=dev, dtype=torch.long)
