@@ -24,7 +24,10 @@ replay costs the real context, not ``t_max``.
 
 from __future__ import annotations
 
-from collections.abc import Callable, Sequence
+import contextlib
+import gc
+import threading
+from collections.abc import Callable, Iterator, Sequence
 from dataclasses import dataclass
 
 import numpy as np
@@ -168,6 +171,34 @@ def _fill_inputs(out: DecodeInputs, block_tables: Sequence[Sequence[int]], num_c
     torch.autograd.graph.increment_version([getattr(out, n) for n in DecodeInputs.__slots__])
 
 
+_gc_lock = threading.Lock()
+_gc_captures = 0  # captures under way
+_gc_enabled = False  # whether the first of them found the collector on
+
+
+@contextlib.contextmanager
+def capturing(graph: torch.cuda.CUDAGraph, pool=None) -> Iterator[None]:
+    """``torch.cuda.graph`` with Python's automatic garbage collection held off. A
+    collection may find another graph in a reference cycle (a dropped decoder whose
+    step function refers to it); a graph's destructor waits for the device, which
+    is an error while a stream is capturing, and an error in a destructor ends the
+    process."""
+    global _gc_captures, _gc_enabled
+    with _gc_lock:
+        if _gc_captures == 0:
+            _gc_enabled = gc.isenabled()
+            gc.disable()
+        _gc_captures += 1
+    try:
+        with torch.cuda.graph(graph) if pool is None else torch.cuda.graph(graph, pool=pool):
+            yield
+    finally:
+        with _gc_lock:
+            _gc_captures -= 1
+            if _gc_captures == 0 and _gc_enabled:
+                gc.enable()
+
+
 @dataclass(slots=True)
 class _Captured:
     graph: torch.cuda.CUDAGraph
@@ -263,12 +294,7 @@ class HipGraphDecoder:
                 self._forward(buf)
         torch.cuda.current_stream(self.device).wait_stream(stream)
         graph = torch.cuda.CUDAGraph()
-        ctx = (
-            torch.cuda.graph(graph)
-            if self._mempool is None
-            else torch.cuda.graph(graph, pool=self._mempool)
-        )
-        with ctx:
+        with capturing(graph, self._mempool):
             out = self._forward(buf)
         if self._mempool is None:
             self._mempool = graph.pool()

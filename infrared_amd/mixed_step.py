@@ -41,6 +41,7 @@ from dataclasses import dataclass
 import torch
 
 from infrared_amd import kernels, metadata
+from infrared_amd.hip_graph import capturing
 from infrared_amd.paged_kv_cache import PagedKVPool
 
 
@@ -265,7 +266,7 @@ class MixedStep:
                 self.eager()
         torch.cuda.current_stream(self.pool.device).wait_stream(stream)
         graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(graph):
+        with capturing(graph):
             self.eager()
         self._graph = graph
 

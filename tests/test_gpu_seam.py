@@ -4,6 +4,7 @@ pool's write/gather surface, and hipGraph capture/replay of a decode step."""
 
 from __future__ import annotations
 
+import gc
 from dataclasses import dataclass
 
 import pytest
@@ -915,6 +916,7 @@ def test_reference_form_check_sees_refilled_graph_buffers():
 
     def step(buf, paged):
         bufs["now"] = buf
+        assert gc.isenabled() != torch.cuda.is_current_stream_capturing()  # held off in a capture
         return paged_attention(q, k, v, _ReferenceContext(pool, buf.write_slots, buf.gather_slots), buf.mask, 0,
                                d**-0.5, n_rep)
 

@@ -5,6 +5,8 @@ and the oracle's loop restatements."""
 from __future__ import annotations
 
 import contextlib
+import gc
+import threading
 
 import numpy as np
 import pytest
@@ -293,3 +295,66 @@ def test_step_metadata_is_built_on_its_own_device(call, monkeypatch):
     else:
         metadata.prefill_context(type("Pool", (), {"device": cpu, "block_size": 16})(), [[1]], [3], [2])
     assert calls == [[cpu]] and not current
+
+
+def test_no_graph_is_collected_during_a_capture(monkeypatch):
+    """Graphs in dropped reference cycles (a state, its decoder, its step function) are
+    not destroyed by an automatic collection while another one is captured: their
+    destructors wait for the device. The collector is back on afterwards, whatever
+    happened inside, and only after the last of several captures; if it was off it
+    stays off."""
+    under = {"capture": False}
+    destroyed = []
+
+    class Graph:
+        def __del__(self):
+            destroyed.append(under["capture"])
+
+    @contextlib.contextmanager
+    def graph(g, **kwargs):
+        under["capture"] = True
+        yield
+        under["capture"] = False
+
+    monkeypatch.setattr(torch.cuda, "graph", graph)
+    pool = type("Pool", (), {"device": torch.device("cpu"), "dtype": torch.float32})()
+    enabled = gc.isenabled()
+    gc.enable()
+    try:
+        for _ in range(20):
+            state = {}
+            state["decoder"] = hip_graph.HipGraphDecoder(None, pool, max_num_seqs=1, t_max=8, block_size=8,
+                                                         step_fn=lambda buf, paged, s=state: s)
+            state["graph"] = Graph()
+            del state
+            with hip_graph.capturing(None):
+                assert not gc.isenabled()
+                keep = [[i] for i in range(3000)]  # enough objects to set a collection off
+            assert gc.isenabled()
+            del keep
+        gc.collect()
+        assert len(destroyed) == 20 and not any(destroyed)
+        with pytest.raises(KeyError), hip_graph.capturing(None):
+            raise KeyError
+        assert gc.isenabled()
+        inside, leave = threading.Event(), threading.Event()
+
+        def other():
+            with hip_graph.capturing(None):
+                inside.set()
+                leave.wait(10)
+
+        t = threading.Thread(target=other)
+        with hip_graph.capturing(None):
+            t.start()
+            assert inside.wait(10)
+        assert not gc.isenabled()  # the other capture is still under way
+        leave.set()
+        t.join()
+        assert gc.isenabled()
+        gc.disable()
+        with hip_graph.capturing(None):
+            pass
+        assert not gc.isenabled()
+    finally:
+        (gc.enable if enabled else gc.disable)()
