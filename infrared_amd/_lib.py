@@ -161,6 +161,7 @@ def lib() -> ctypes.CDLL:
 
 
 _seam = None
+_HERE = contextlib.nullcontext()
 
 
 def seam():
@@ -189,7 +190,9 @@ def stream_of(t: torch.Tensor) -> int:
 def on_device(device: torch.device):
     """Context in which a call launches on ``device``, whichever is current (its
     stream's raw handle may be the null stream, which is the current device's)."""
-    return torch.cuda.device(device) if device.type == "cuda" else contextlib.nullcontext()
+    if device.type != "cuda" or device.index == torch.cuda.current_device():
+        return _HERE
+    return torch.cuda.device(device)
 
 
 def check(rc: int, what: str) -> None:

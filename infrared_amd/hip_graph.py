@@ -137,14 +137,15 @@ def _check_rows(num_cached: Sequence[int], last_tokens: Sequence[int], bucket_b:
     b = len(last_tokens)
     if not 0 < b <= bucket_b:
         raise ValueError(f"need 0 < b ({b}) <= bucket_b ({bucket_b})")
-    cached = host_list(num_cached)
-    cached = [int(cached[j]) for j in range(b)]  # (IndexError if one is missing)
+    cached = list(map(int, host_list(num_cached)[:b]))
+    if len(cached) < b:
+        raise IndexError(f"{len(cached)} cached lengths for {b} rows")
     for n in cached:
         if n < 0:
             raise ValueError(f"num_cached {n} is negative")
         if n + 1 > t_max:
             raise ValueError(f"context_len {n + 1} exceeds t_max {t_max}")
-    return cached, [int(t) for t in host_list(last_tokens)]
+    return cached, list(map(int, host_list(last_tokens)))
 
 
 def _fill_inputs(out: DecodeInputs, block_tables: Sequence[Sequence[int]], num_cached: list[int],

@@ -168,10 +168,11 @@ def prefill_context(
     bs = pool.block_size
     if not (len(block_tables) == len(num_cached) == len(q_lens)):
         raise ValueError("block_tables, num_cached and q_lens must have one entry per sequence")
-    num_cached, q_lens = [[index(n) for n in host_list(x)] for x in (num_cached, q_lens)]
+    num_cached, q_lens = list(map(index, host_list(num_cached))), list(map(index, host_list(q_lens)))
     lengths = [c + n for c, n in zip(num_cached, q_lens)]
-    width = max(blocks_for(n, bs) for n in lengths) if lengths else 0
-    rows = [r[: max(width, 1)] for r in block_tables]
+    width = blocks_for(max(lengths), bs) if lengths else 0
+    cut = max(width, 1)
+    rows = [r[:cut] for r in block_tables]
     total, n = sum(q_lens), len(q_lens)
     if min(q_lens, default=0) < 0:
         raise ValueError("q_lens must not be negative")
