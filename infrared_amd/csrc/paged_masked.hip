@@ -98,15 +98,20 @@ __device__ __forceinline__ int64_t part_row(const MaskedArgs& a, int part, int b
 // fp32 call, and masks whose key stride is not 1: one workgroup of 4 wavefronts
 // per (sequence, KV head, 16 columns, part of the keys), a wavefront taking
 // 16-key tiles round-robin. What bounds it is latency: a tile's K and V
-// addresses come from slots that are loaded first. So a wavefront keeps the
-// next tile's K, V and mask loads and the slots of the tile after that in
-// flight behind the tile being computed, each slot loaded once per key and
-// handed to the lanes that need it, and the keys are cut into parts when the
-// call has too few workgroups for the CUs (two per CU fit). 24 sequences of up to
-// 2048 keys, 28/4 heads of 128, bf16: 17.5 + 3.9 us (merge) against 107 us for one
-// part, one tile at a time and four slot loads a lane; 4 workgroups per CU: 33.8 us.
+// addresses come from slots that are loaded first. So a wavefront keeps the slots
+// of the next tile in flight behind the tile being computed, each slot loaded once
+// per key and handed to the lanes that need it, and the keys are cut into parts
+// when the call has too few workgroups for the CUs (two per CU fit). 24 sequences of
+// up to 2048 keys, 28/4 heads of 128, bf16: 17.5 + 3.9 us (merge) against 107 us for
+// one part, one tile at a time and four slot loads a lane; 4 workgroups per CU: 33.8 us.
+// 16-bit calls also keep the next tile's K, V and mask loads in flight, which gives
+// what large batches have to gain (64 sequences x 2048 keys: 50.2 against 53.5 us with
+// 8 KV heads of 64, 48.5 / 49.3 with 4 of 128) and costs small ones 0.2 us. fp32 calls
+// do not: two tiles take 312 registers at head_dim 128, one 164, and with one
+// wavefront a SIMD instead of three 256 tokens x 2048 keys took 193 us against 129,
+// 64 decodes 127 / 103; at head_dim 64 43.8 us against 44.8.
 template <int DT, int D, bool SERIAL>
-__global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(DT == IR_DTYPE_F32 && D == 128 ? 1 : 2)))
+__global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2)))
 void paged_masked_kernel(MaskedArgs a) {
   typedef TileShape<DT, D> Sh;
   constexpr int EB = Sh::EB;
@@ -189,7 +194,17 @@ void paged_masked_kernel(MaskedArgs a) {
     state_init(st);
     t_hi = (int)((int64_t)(p + 1) * ntiles / a.parts);
     int ti = (int)((int64_t)p * ntiles / a.parts) + w;
-    if (a.num_slots > 0 && ti < t_hi) {
+    if constexpr (DT == IR_DTYPE_F32) {
+      if (a.num_slots > 0) {
+        int64_t s = load_slot(ti);
+        for (; ti < t_hi; ti += kWaves) {
+          Loads x;
+          issue(ti, s, x);
+          s = load_slot(ti + kWaves);
+          compute(x);
+        }
+      }
+    } else if (a.num_slots > 0 && ti < t_hi) {
       Loads x, y;
       issue(ti, load_slot(ti), x);
       int64_t s_next = load_slot(ti + kWaves);
