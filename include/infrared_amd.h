@@ -71,8 +71,8 @@ enum {
   IR_FORM_CLEAR_ON_FAIL = 1 /* after the check, set every context length to 0 when *bad is set */
 };
 
-/* ir_paged_attention_masked: (query token, head) columns per KV head up to which a call runs the
-   kernel for few columns; gated by run_if, such a call is one launch and uses no workspace */
+/* ir_paged_attention_masked: (query token, head) columns per KV head up to which every call runs
+   the kernel for few columns; gated by run_if, such a call is one launch and uses no workspace */
 enum { IR_MASKED_FEW_COLUMNS = 32 };
 
 /* Message of the last failed call on this thread ("" if none). */

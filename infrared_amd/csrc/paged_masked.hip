@@ -94,8 +94,8 @@ __device__ __forceinline__ int64_t part_row(const MaskedArgs& a, int part, int b
 
 // ---------------------------------------------------------------- few columns, or fp32
 //
-// Decode batches and anything else with at most 32 columns per KV head, every
-// fp32 call, and masks whose key stride is not 1: one workgroup of 4 wavefronts
+// Decode batches and anything else with at most 32 columns per KV head, short
+// frames, every fp32 call, and masks whose key stride is not 1: one workgroup of 4 wavefronts
 // per (sequence, KV head, 16 columns, part of the keys), a wavefront taking
 // 16-key tiles round-robin. What bounds it is latency: a tile's K and V
 // addresses come from slots that are loaded first. So a wavefront keeps the slots
@@ -888,6 +888,8 @@ __global__ __launch_bounds__(256) void paged_masked_merge_kernel(MaskedArgs a) {
 // ---------------------------------------------------------------- host side
 
 constexpr int kSurveyParts = 12;
+constexpr int kFewKeys = 320;          // a frame of at most these keys,
+constexpr int64_t kFewKeysAll = 8192;  // and these over all sequences and KV heads, may take the 16-column kernel
 constexpr int64_t kMaxPartBytes = 256ll << 20;  // bound of a call's partial rows
 
 struct Split {
@@ -903,17 +905,24 @@ struct Split {
 // workgroup: up to 16 the 16-column kernel is 1.2-1.5x faster (24 sequences x 2048
 // keys, 4 KV heads of 128, bf16, 14 columns: 24.8 us against 35.6 wide), 17 to 32
 // tie (28 columns: 40.6 / 36.8; one sequence of 4096: 14.1 / 17.1), and from 33 its
-// third pass over the keys loses (35 columns, 64 sequences x 2048: 137 / 75.8).
+// third pass over the keys loses (35 columns, 64 sequences x 2048: 137 / 75.8). With
+// few keys, though, that pass costs nothing and the shorter chain of the 16-column
+// kernel wins while its workgroups are resident at once (28/4 heads of 128, us on
+// 16 columns / wide: 40 tokens x 40 keys 5.7 / 8.8, 100 x 128 7.7 / 11.3, 256 x 256
+// 13.9 / 17.9; 320 x 320, 560 workgroups: 23.2 / 21.9; 16 sequences of 5 x 256, 16K
+// keys in all: 14.3 / 13.4; 100 x 512: 17.6 / 16.8).
 Split split_of(int64_t batch, int64_t seq_q, int64_t seq_k, int num_q_heads, int num_kv_heads, int head_dim,
                int dtype, int mask_dtype, int64_t mask_t_stride, int64_t num_slots) {
   const int n_rep = num_q_heads / num_kv_heads;
   const int64_t rows = seq_q * n_rep;
   Split s;
-  s.wide = rows > IR_MASKED_FEW_COLUMNS && dtype != IR_DTYPE_F32 &&
+  const int64_t slots = (int64_t)device_cus() * 2;
+  const bool few_keys = seq_k <= kFewKeys && batch * num_kv_heads * seq_k <= kFewKeysAll &&
+                        batch * num_kv_heads * ((rows + 15) / 16) <= slots;
+  s.wide = rows > IR_MASKED_FEW_COLUMNS && !few_keys && dtype != IR_DTYPE_F32 &&
            (mask_dtype == dtype || mask_dtype == IR_DTYPE_F32) && mask_t_stride == 1 && seq_k <= (1 << 28) &&
            num_slots <= 0x7fffffff;
   const int64_t nt = (seq_k + kTileKeys - 1) / kTileKeys, n_rtw = (rows + kWideCols - 1) / kWideCols;
-  const int64_t slots = (int64_t)device_cus() * 2;
   s.nwg = batch * num_kv_heads * (s.wide ? n_rtw : (rows + 15) / 16);
   // The survey reads all keys and the mask once, a launch of ~10 us or one column
   // block's walk, whichever is more, and the walks another ~8: it can pay where

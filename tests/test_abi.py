@@ -157,6 +157,18 @@ def test_masked_workspace_covers_a_survey_only_where_one_launch_holds_it():
     assert size(250, *args) > 250 * 32 * 1024 * 4  # at least a bound per key tile and KV head
 
 
+def test_masked_short_frames_take_the_kernel_for_few_columns():
+    """Up to 320 keys, 8192 over all sequences and KV heads, and 512 workgroups of 16
+    columns: by the parts the workspace holds on both sides of each line. Over 256
+    workgroups of 16 columns take one part (no workspace); the wide kernel, with an eighth
+    of the workgroups, one for every two of its 64-key tiles."""
+    for b, sq, t, kv, few in ((1, 146, 256, 8, True), (1, 147, 256, 8, False), (1, 146, 320, 8, True),
+                              (1, 146, 321, 8, False), (4, 36, 256, 8, True), (4, 36, 257, 8, False)):
+        size = _lib.lib().ir_paged_attention_masked_workspace_size(
+            b, sq, t, kv * 7, kv, 128, _lib.DTYPE_BF16, _lib.DTYPE_BF16, 1)
+        assert size == (0 if few else (-(-t // 64) // 2) * b * sq * kv * 7 * 130 * 4), (b, sq, t, kv)
+
+
 def test_masked_survey_needs_blocks_and_tiles():
     """A surveyed call has 12 blocks of 128 columns a sequence, and 8 key tiles (11 at
     head_dim 64) for each of the 512 workgroups the device holds: the workspace on both

@@ -489,13 +489,17 @@ def test_masked_fully_masked_row_is_uniform_and_bad_slot_flagged():
     (1, 4, 1, 4, 7, 128, torch.bfloat16, torch.bfloat16),     # 28 columns: the narrow kernel, one key
     (3, 1, 1003, 2, 7, 64, torch.float32, torch.float32),     # split, ragged last 16 keys
     (2, 1, 2048, 4, 7, 128, torch.float16, torch.float32),    # split, whole tiles
-    (1, 5, 63, 4, 7, 128, torch.bfloat16, torch.bfloat16),    # 35 columns: the wide kernel, one ragged tile
-    (1, 19, 64, 4, 7, 128, torch.float16, torch.float16),     # 133 columns: a second workgroup of 5
+    (1, 5, 63, 4, 7, 128, torch.bfloat16, torch.bfloat16),    # 35 columns, few keys: the narrow kernel
+    (40, 5, 63, 4, 7, 128, torch.bfloat16, torch.bfloat16),   # 40 such sequences: the wide kernel, one ragged tile
+    (40, 19, 64, 4, 7, 128, torch.float16, torch.float16),    # 133 columns: a second workgroup of 5
+    (1, 292, 320, 4, 7, 64, torch.bfloat16, torch.bfloat16),  # 512 narrow workgroups, the most keys: the narrow kernel
+    (1, 293, 320, 4, 7, 64, torch.bfloat16, torch.bfloat16),  # 516: the wide kernel
+    (1, 40, 321, 4, 7, 64, torch.float16, torch.float16),     # one key more: the wide kernel
     (1, 40, 577, 2, 7, 64, torch.bfloat16, torch.bfloat16),   # split wide, ragged, head_dim 64
     (2, 37, 700, 4, 7, 128, torch.bfloat16, torch.float32),   # fp32 mask read per lane
     (1, 70, 321, 2, 4, 128, torch.bfloat16, torch.bfloat16),  # 4 heads a token: 16-bit mask read per lane
-    (1, 130, 200, 1, 1, 64, torch.float16, torch.float16),    # one head a token
-    (1, 27, 130, 1, 5, 128, torch.bfloat16, torch.bfloat16),  # 5 heads: 27 tokens in a workgroup
+    (48, 130, 200, 1, 1, 64, torch.float16, torch.float16),   # one head a token
+    (64, 27, 130, 1, 5, 128, torch.bfloat16, torch.bfloat16), # 5 heads: 27 tokens in a workgroup
     (1, 9, 4200, 1, 40, 64, torch.bfloat16, torch.bfloat16),  # 40 heads a token
     (2, 40, 1100, 2, 7, 128, torch.float16, torch.float16),   # two sequences
     (2, 250, 1100, 10, 7, 128, torch.float16, torch.float16), # two sequences, surveyed
