@@ -1213,6 +1213,7 @@ struct PlanArgs {
   int64_t bt_stride;
   int num_seqs, total_q, n_qblocks, tq, cap, bs;  // cap: keys the block tables hold
   int num_kv_heads, slots, cap_pieces, xcds;      // slots: workgroups whose mean load is the cut threshold
+  int slack;          // nothing is cut if no item is further than this over the threshold
   int share_groups;   // place share groups on slots of XCDs (else one global order)
   int entries;        // workgroups of a planned call
   int2* items;        // [entries]
@@ -1346,6 +1347,7 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(PlanArgs a) 
   // (it usually fits as it is: one count instead of a bisection's five or six,
   // ~1 us each: 11.4 us a plan against 15.4 on 6 fp32 chunks, 14/2 heads)
   int lo = (int)max((int64_t)kMinPieceTiles, (total * H * 3 + 2 * a.slots - 1) / (2 * a.slots));
+  if (wmax <= lo + a.slack) lo = max(lo, wmax);
   int hi = max(lo, wmax);
   for (int mid = lo; lo < hi; mid = lo + (hi - lo) / 2) {
     int64_t cnt = 0;
@@ -1550,7 +1552,11 @@ PrefillGeometry prefill_geometry(int max_q_len, int n_rep) {
 // loads, so at 64 the plan cuts for three (6 chunks of 64..512 tokens after up to
 // 1500, 14/2 heads, per layer: 63.8 us against 66.1 cut for two; cut for four
 // 64.6, as the pieces then exceed the plan's capacity and the threshold rises
-// again). The capacity stays that of two per CU.
+// again; one chunk of 512 after 16,000 tokens 315 against 417). The capacity stays
+// that of two per CU. Items that exceed this lower threshold by no more than a
+// piece's fixed cost are better whole: 8 chunks of 512 after 4096, 8 heads, 512
+// items of 65..72 tiles at a threshold of 69: 344 us whole, 385 cut. Over 75 frames
+// two mixes of 4 and 5 chunks stay 6 and 9% slower than cut for two.
 PrefillGeometry prefill_geometry_f32(int max_q_len, int n_rep, int head_dim) {
   PrefillGeometry g;
   g.nw = 4;
@@ -1828,6 +1834,7 @@ extern "C" int ir_paged_prefill_plan(const int32_t* cu_seqlens_q, const int32_t*
   p.bs = block_size;
   p.num_kv_heads = num_kv_heads;
   p.slots = geo.cut_slots;
+  p.slack = geo.cut_slots > geo.slots ? kPieceFixed : 0;
   p.cap_pieces = prefill_knobs().cuts ? (int)ly.cap_pieces : 0;
   p.xcds = plan_xcds();
   p.share_groups = (flags & IR_PLAN_SHARE_GROUPS) != 0;

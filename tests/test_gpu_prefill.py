@@ -213,6 +213,19 @@ def test_prefill_fp32_reloads_block_ids_and_runs_its_plan():
         _check_f32(case, plan16)
 
 
+@pytest.mark.parametrize("n,q_len,prefix,cut", [(8, 512, 4096, False), (8, 512, 3584, False), (1, 4096, 0, True)])
+def test_fp32_plan_leaves_even_items_whole(n, q_len, prefix, cut):
+    """head_dim 64, 8 single heads, 512 items of 64 tokens. After a long prefix they weigh
+    prefix / 64 + 1 .. + 8 tiles, at most 3 more than the threshold (1.5 times the mean load
+    of 768 workgroups): none is cut. One chunk of 4096 has items of 1 .. 64: some are."""
+    blocks = (prefix + q_len) // 16
+    cu = torch.arange(n + 1, dtype=torch.int32, device=DEV) * q_len
+    q_start = torch.full((n,), prefix, dtype=torch.int32, device=DEV)
+    bt = torch.arange(n * blocks, dtype=torch.int32, device=DEV).view(n, blocks)
+    plan = kernels.prefill_plan(cu, q_start, bt, n * q_len, q_len, 16, 8, 8, 64, dtype=torch.float32)
+    assert (max(_cut_entries(plan, 512)) > 1) == cut
+
+
 def test_prefill_fp32_planned_long_prefixes():
     """fp32 chunks after long prefixes that pairs share, and an empty chunk, on
     a plan: cut items merged within 1e-4 of the restatement, and a plan
